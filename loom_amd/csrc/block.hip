@@ -2628,8 +2628,6 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const float* __restrict__ 
     extern __shared__ float xs[];  // hidden
     const int tid = threadIdx.x;
     const int v0 = blockIdx.x * kHeadLogits;
-    x += (size_t)blockIdx.y * hidden;
-    logits += (size_t)blockIdx.y * vocab;
     for (int i = tid; i < hidden; i += 256) xs[i] = x[i];
     constexpr int C4N = kHeadSlab / 4;           // threads per row segment
     constexpr int NL = kHeadLogits * C4N / 256;  // float4 loads per thread per slab
@@ -2707,13 +2705,206 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const float* __restrict__ 
     if (v0 + tid < vocab) logits[v0 + tid] = (float)r;
 }
 
+// The same logits for several rows, on the fp64 matrix cores.  Measured on
+// gfx950 (random, wide-range, cancelling, infinite and NaN operands, five
+// million outputs): v_mfma_f64_16x16x4f64 rounds after each of its four
+// products, k = 0, 1, 2, 3, exactly as four FMAs in that order.  The product
+// of two fp32 values is exact in fp64, so a chain of these MFMAs is loom's
+// chain bit for bit once consecutive k hold the chain's consecutive terms:
+//  - DOTTILE: chain l takes column 8 c + l of chunk c, so lane (r, g) holds
+//    chunk 4 s + g of table row r (32 contiguous bytes) at step s and its
+//    eight floats feed the eight chains; the tree and the n%8 tail follow per
+//    output, in one lane;
+//  - sequential: k = g takes column 4 m + g (one dword a lane).
+// A wave owns 16 vocab rows (B) and 16 MT rows of x (A), 256 threads four
+// such waves; x goes through LDS in slabs of 128 columns (pitch 132: the 16
+// rows that a 16-byte read covers fall in distinct banks), the table straight
+// to registers, four steps ahead of their MFMAs (2 KB a wave and step: 96 KB
+// in flight a CU at three waves per SIMD).  The barriers wait for LDS only, so
+// the table loads stay in flight across them.
+// Bound: HBM for one 16-row tile (1.31 GB at vocab 128256 x 2560: 195 us at
+// the 6.7 TB/s of the one-row kernel; 145 us of MFMA issue): 2 to 16 rows take
+// 302-315 us, against 195 us a row (16 rows 3,066 us) with the one-row kernel
+// reading the table once per row.  MT = 2 from 17 rows (the table read once
+// for 32 rows, 409 us; two MT = 1 tiles would take twice 302).  Sequential order:
+// 655-673 us (its one chain per output waits on every MFMA).
+// Padding columns are zero in both operands (0 * Inf never arises; a chain
+// starts at +0 and so never holds -0, which + 0 would change); rows past
+// `rows` and vocab rows past the table are computed and not stored.
+// ------------------------------------------------------------------------
+
+typedef double v4d_head __attribute__((ext_vector_type(4)));
+constexpr int kHeadCols = 128;            // columns per x slab: four steps of 32
+constexpr int kHeadPitch = kHeadCols + 4;
+constexpr int kHeadAhead = 4;             // table steps in flight
+
+template <bool VEC, bool DOTTILE, int MT>
+__global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restrict__ table, int vocab, int hidden,
+                                                           const float* __restrict__ x, int rows,
+                                                           float* __restrict__ logits) {
+    static_assert(kHeadCols == 32 * kHeadAhead, "a slab is one turn of the table ring");
+    __shared__ __align__(16) float xs[2][16 * MT * kHeadPitch];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r = lane & 15, g = lane >> 4;
+    const int v0 = (blockIdx.x * 4 + wave) * 16;
+    const int row0 = blockIdx.y * 16 * MT;
+    // raw buffers over the wave's table rows and the workgroup's x rows: loads
+    // past a buffer's end read 0 with no branch (a branch around a load would
+    // wait for the table loads in flight)
+    const __amdgpu_buffer_rsrc_t wres =
+        buffer_rsrc(table + (size_t)min(v0, vocab - 1) * hidden, (uint32_t)max(min(vocab - v0, 16), 1) * hidden * 4u);
+    const __amdgpu_buffer_rsrc_t xres =
+        buffer_rsrc(x + (size_t)row0 * hidden, (uint32_t)min(rows - row0, 16 * MT) * hidden * 4u);
+    constexpr uint32_t kPast = 0x7fffffffu & ~15u;
+    // columns that the chains take (DotTile: whole 8-column chunks), whole
+    // slabs of them, and the steps of 32 columns after those
+    const int ncols = DOTTILE ? hidden & ~7 : hidden;
+    const int nslab = ncols / kHeadCols;
+    const int nrest = (ncols - nslab * kHeadCols + 31) / 32;
+
+    // this thread's slots of an x slab: row tid/32 + 8 i, columns 4 (tid%32) ..
+    constexpr int NX = 2 * MT;
+    const int xr0 = tid >> 5, xc = (tid & 31) * 4;
+    uint32_t xn[NX][4];
+    auto load_x = [&](int c0) {
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {
+            const int c = c0 + xc;
+            const uint32_t off = (uint32_t)((xr0 + 8 * i) * hidden + c) * 4u;
+            if constexpr (VEC) {
+                const uint4 q = buffer_load16(xres, c < ncols ? off : kPast);
+                xn[i][0] = q.x, xn[i][1] = q.y, xn[i][2] = q.z, xn[i][3] = q.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    xn[i][e] = __builtin_amdgcn_raw_buffer_load_b32(xres, (int)(c + e < ncols ? off + 4u * e : kPast), 0, 0);
+            }
+        }
+    };
+    auto store_x = [&](float* buf) {
+#pragma unroll
+        for (int i = 0; i < NX; ++i)
+            *(uint4*)&buf[(xr0 + 8 * i) * kHeadPitch + xc] = make_uint4(xn[i][0], xn[i][1], xn[i][2], xn[i][3]);
+    };
+    // the eight table values of this lane for the step at column c0: chunk g
+    // (DotTile), or columns 4 m + g (sequential); columns past ncols read 0
+    const int wv = (r * hidden + (DOTTILE ? 8 * g : g)) * 4;
+    auto load_w = [&](int c0, uint32_t (&w)[8], auto guard) {
+        if constexpr (DOTTILE && VEC && !decltype(guard)::value) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const uint4 a = __builtin_bit_cast(
+                    uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, wv + 16 * q, c0 * 4, kLoadNT));
+                w[4 * q] = a.x, w[4 * q + 1] = a.y, w[4 * q + 2] = a.z, w[4 * q + 3] = a.w;
+            }
+        } else {
+#pragma unroll
+            for (int l = 0; l < 8; ++l) {
+                const int e = DOTTILE ? l : 4 * l;
+                const bool past = decltype(guard)::value && c0 + e + (DOTTILE ? 8 * g : g) >= ncols;
+                w[l] = __builtin_amdgcn_raw_buffer_load_b32(wres, past ? (int)kPast : wv + 4 * (c0 + e), 0, 0);
+            }
+        }
+    };
+    constexpr int NC = DOTTILE ? 8 : 1;
+    v4d_head acc[NC][MT];
+#pragma unroll
+    for (int l = 0; l < NC; ++l)
+#pragma unroll
+        for (int t = 0; t < MT; ++t) acc[l][t] = v4d_head{0.0, 0.0, 0.0, 0.0};
+    auto step = [&](const float* buf, int cs, const uint32_t (&w)[8]) {
+#pragma unroll
+        for (int t = 0; t < MT; ++t) {
+            const float* xb = buf + (16 * t + r) * kHeadPitch + cs;
+            float a[8];
+            if (DOTTILE) {
+                const float4 p = *(const float4*)(xb + 8 * g), q = *(const float4*)(xb + 8 * g + 4);
+                a[0] = p.x, a[1] = p.y, a[2] = p.z, a[3] = p.w, a[4] = q.x, a[5] = q.y, a[6] = q.z, a[7] = q.w;
+            } else {
+#pragma unroll
+                for (int l = 0; l < 8; ++l) a[l] = xb[4 * l + g];
+            }
+#pragma unroll
+            for (int l = 0; l < 8; ++l)
+                acc[DOTTILE ? l : 0][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    (double)a[l], (double)__uint_as_float(w[l]), acc[DOTTILE ? l : 0][t], 0, 0, 0);
+        }
+    };
+
+    uint32_t ring[kHeadAhead][8];
+    load_x(0);
+    if (nslab > 0) {
+#pragma unroll
+        for (int k = 0; k < kHeadAhead; ++k) load_w(32 * k, ring[k], std::false_type{});
+    }
+    store_x(xs[0]);
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    for (int i = 0; i < nslab; ++i) {
+        const int c0 = i * kHeadCols;
+        const float* buf = xs[i & 1];
+        load_x(c0 + kHeadCols);  // (all zero past the last column)
+        // the last slab loads its own columns again rather than branch
+        const int cn = i + 1 < nslab ? c0 + kHeadCols : c0;
+#pragma unroll
+        for (int k = 0; k < kHeadAhead; ++k) {
+            step(buf, 32 * k, ring[k]);
+            load_w(cn + 32 * k, ring[k], std::false_type{});
+        }
+        store_x(xs[(i & 1) ^ 1]);  // last read before the previous barrier
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        __builtin_amdgcn_s_barrier();
+    }
+    for (int k = 0; k < nrest; ++k) {
+        uint32_t w[8];
+        load_w(nslab * kHeadCols + 32 * k, w, std::true_type{});
+        step(xs[nslab & 1], 32 * k, w);
+    }
+
+    // element u of lane (r, g): x row 4 u + g of the tile, vocab row v0 + r
+    const int v = v0 + r;
+#pragma unroll
+    for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int row = row0 + 16 * t + 4 * u + g;
+            if (row >= rows || v >= vocab) continue;
+            double s = acc[0][t][u];
+            if constexpr (DOTTILE) {
+                s = (((acc[0][t][u] + acc[4][t][u]) + (acc[2][t][u] + acc[6][t][u])) +
+                     ((acc[1][t][u] + acc[5][t][u]) + (acc[3][t][u] + acc[7][t][u]))) + 0.0;
+                for (int c = ncols; c < hidden; ++c) 
+                    s = fma((double)x[(size_t)row * hidden + c], (double)table[(size_t)v * hidden + c], s);
+            }
+            logits[(size_t)row * vocab + v] = (float)s;
+        }
+}
+
 template <bool DOTTILE>
 static hipError_t launch_head(const float* table, int vocab, int hidden, const float* x, int rows,
                               float* logits, hipStream_t s) {
     if (vocab <= 0 || hidden <= 0 || rows <= 0) return hipSuccess;
     const size_t shm = (size_t)hidden * sizeof(float);
     if (shm > 64 * 1024) return hipErrorInvalidValue;
-    const dim3 g((unsigned)ceil_div(vocab, kHeadLogits), rows), b(256);
+    const dim3 b(256);
+    if (rows > 1) {
+        const bool vec = hidden % 8 == 0 && (((uintptr_t)table | (uintptr_t)x) & 15) == 0;
+        const int mt = rows > 16 ? 2 : 1;
+        const dim3 g((unsigned)ceil_div(vocab, 64), (unsigned)ceil_div(rows, 16 * mt));
+#define LAMD_HEAD_ROWS(V, MTV)                                                                            \
+    hipLaunchKernelGGL((lm_head_rows_kernel<V, DOTTILE, MTV>), g, b, 0, s, table, vocab, hidden, x, rows, \
+                       logits)
+        if (mt == 2) {
+            if (vec) LAMD_HEAD_ROWS(true, 2);
+            else LAMD_HEAD_ROWS(false, 2);
+        } else {
+            if (vec) LAMD_HEAD_ROWS(true, 1);
+            else LAMD_HEAD_ROWS(false, 1);
+        }
+#undef LAMD_HEAD_ROWS
+        return hipGetLastError();
+    }
+    const dim3 g((unsigned)ceil_div(vocab, kHeadLogits));
     if (hidden % 4 == 0 && ((uintptr_t)table & 15) == 0) {
         hipLaunchKernelGGL((lm_head_kernel<true, DOTTILE>), g, b, shm, s, table, vocab, hidden, x,
                            logits);

@@ -787,6 +787,12 @@ void loom_amd_model_release(loom_amd_model* m) {
     if (m) free_model(m);
 }
 
+// Rows that the screened greedy head takes one after another (about 78 us a
+// row at vocab 128256 x 2560, 38 us at 32000); above, the full head of all
+// rows in one pass over the table is shorter (302 us and 76 us for 2 to 16
+// rows, sequential order 655 us).
+constexpr int kScreenMaxRows = 3;
+
 // Final norm + LM head + argmax of each sequence's last row (row stride ld
 // floats between sequences), writing the token at *pos + offset.
 static int model_head(loom_amd_model* m, const float* last, long ld, int batch, int offset,
@@ -826,7 +832,7 @@ static int model_head(loom_amd_model* m, const float* last, long ld, int batch, 
             }
         }
         if (e != hipSuccess) return fail_hip("model ternary lm head", e);
-    } else if (m->lm_q && tune_int("LOOM_AMD_LM_SCREEN", 1) != 0) {
+    } else if (m->lm_q && batch <= kScreenMaxRows && tune_int("LOOM_AMD_LM_SCREEN", 1) != 0) {
         // greedy pick from an int8 screening pass and the candidates' exact
         // logits, one row after the other (the bounds and the threshold are
         // per row; every call leaves the threshold cleared)

@@ -907,3 +907,29 @@ def test_model_sequential_lm_head(orc, torch_dev, tf):
     for b in range(2):
         assert step_logits[b].tobytes() == orc.lm_head(hid[b], M.emb, simd=False).tobytes()
     model.release()
+
+
+@pytest.mark.parametrize("sequential", [False, True])
+@pytest.mark.parametrize("rows,vocab,hidden,skip", [(2, 65, 32, 0), (16, 63, 136, 0), (17, 130, 260, 0), (33, 64, 257, 0),
+                                                    (5, 1, 9, 0), (4, 300, 512, 1), (18, 999, 520, 4)])
+def test_lm_head_rows_equal_single_rows(torch_dev, tf, sequential, rows, vocab, hidden, skip):
+    # the several-row head (fp64 matrix cores) gives the one-row kernel's bits:
+    # row tiles of 16 and 32, ragged columns and vocab tiles, a table and rows
+    # off 16-byte alignment (skip floats), wide exponents, NaN and Inf entries
+    torch = torch_dev
+    g = torch.Generator(device="cuda").manual_seed(rows * 1000 + hidden)
+
+    def wide(n):
+        e = torch.randint(-40, 40, (n,), device="cuda", generator=g).float()
+        return torch.randn(n, device="cuda", generator=g) * torch.exp2(e)
+
+    flat = wide(vocab * hidden + skip)
+    flat[-1], flat[skip] = float("inf"), float("nan")
+    table = flat[skip:].view(vocab, hidden)
+    x = wide(rows * hidden + skip)[skip:].view(rows, hidden)
+    x[-1, hidden // 2] = float("-inf")
+    got = tf.lm_head(table, x, sequential)
+    for r in range(rows):
+        one = tf.lm_head(table, x[r:r + 1].clone(), sequential)[0]
+        assert torch.equal(got[r].isnan(), one.isnan()), r
+        assert torch.equal(got[r].nan_to_num(0.5), one.nan_to_num(0.5)), r

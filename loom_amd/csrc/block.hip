@@ -214,12 +214,13 @@ template <int STRICT>
 static hipError_t launch_rmsnorm_t(const float* x, long ldx, int m, int n, const float* gain,
                                    double eps, float* y, int8_t* xq, int ldq, float* amax,
                                    int32_t* xsum, const double* totals, hipStream_t s) {
-    if (xq) {  // (the final norm without quantization keeps the workgroup kernel)
+    {
         const RowNormArgs a{x, ldx, m, n, gain, eps, y, nullptr, xq, ldq, amax, xsum, totals};
         hipError_t e = hipSuccess;
-        if (launch_row_norm_wave(kRowRms, STRICT, a, s, &e)) return e;
+        if (xq && launch_row_norm_wave(kRowRms, STRICT, a, s, &e)) return e;
+        if (launch_row_norm_block(kRowRms, STRICT, a, s, &e)) return e;
     }
-    const size_t shm = STRICT && !totals ? (size_t)ordered_sum_slots(n, 4) * sizeof(double) : 0;
+    const size_t shm = STRICT && !totals ? (size_t)n * sizeof(double) : 0;
     const dim3 g(m), b(256);
 #define LAMD_RMS(VPT)                                                                          \
     hipLaunchKernelGGL((rmsnorm_quant_kernel<STRICT, VPT>), g, b, shm, s, x, ldx, n, gain, eps, y, xq, \
@@ -2534,8 +2535,9 @@ static hipError_t launch_norm_f64_t(double* a, int m, int n, const float* w, dou
         const RowNormArgs ra{a, n, m, n, w, eps, pre, keep ? a : nullptr, xq, ldq, amax, xsum, totals};
         hipError_t e = hipSuccess;
         if (launch_row_norm_wave(kRowInnerF64, STRICT, ra, s, &e)) return e;
+        if (launch_row_norm_block(kRowInnerF64, STRICT, ra, s, &e)) return e;
     }
-    const size_t shm = STRICT && !totals ? (size_t)ordered_sum_slots(n, 4) * sizeof(double) : 0;
+    const size_t shm = STRICT && !totals ? (size_t)n * sizeof(double) : 0;
     const dim3 g(m), b(256);
 #define LAMD_NF64(VPT)                                                                          \
     hipLaunchKernelGGL((norm_quant_f64_kernel<STRICT, VPT>), g, b, shm, s, a, n, w, eps, pre, xq, ldq, \

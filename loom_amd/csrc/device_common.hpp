@@ -370,8 +370,8 @@ __device__ __forceinline__ double readlane_d(double v, int lane) {
 // (squares, exponentials) take the parallel step.
 constexpr int kChainC = 4;  // terms per lane and step of ordered_sum_wave
 
-template <int C>
-__device__ __forceinline__ double ordered_sum_wave(const double* t, int n, double s) {
+template <int C, typename Get>
+__device__ __forceinline__ double ordered_sum_wave_get(Get get, int n, double s) {
     const int lane = threadIdx.x & 63;
     const unsigned long long lt = (1ull << lane) - 1ull;  // lanes below this one
     int base = 0;
@@ -383,7 +383,7 @@ __device__ __forceinline__ double ordered_sum_wave(const double* t, int n, doubl
 #pragma unroll
             for (int i = C - 1; i >= 0; --i) {
                 const int idx = base + lane * C + i;
-                if (idx < n && t[idx] != 0.0) first = i;  // (NaN compares unequal)
+                if (idx < n && get(idx) != 0.0) first = i;  // (NaN compares unequal)
             }
             const unsigned long long nz = __builtin_amdgcn_ballot_w64(first < C);
             if (nz == 0ull) {
@@ -392,13 +392,13 @@ __device__ __forceinline__ double ordered_sum_wave(const double* t, int n, doubl
             }
             const int j = __builtin_ctzll(nz);
             const int idx = base + j * C + __builtin_amdgcn_readlane(first, j);
-            s = s + t[idx];
+            s = s + get(idx);
             base = idx + 1;
             continue;
         }
         if (ex < 56 || ex > 2000) {
             const int end = min(n, base + 64 * C);
-            for (; base < end; ++base) s = s + t[base];
+            for (; base < end; ++base) s = s + get(base);
             continue;
         }
         const double scale = __longlong_as_double((long long)(2098 - ex) << 52);  // 1/q
@@ -411,7 +411,7 @@ __device__ __forceinline__ double ordered_sum_wave(const double* t, int n, doubl
 #pragma unroll
         for (int i = 0; i < C; ++i) {
             const int idx = base + lane * C + i;
-            const double u = (idx < n ? t[idx] : 0.0) * scale;
+            const double u = (idx < n ? get(idx) : 0.0) * scale;
             bad |= !(u >= 0.0 && u < 0x1p52);
             const double fl = floor(u);
             const bool tie = u - fl == 0.5;
@@ -443,11 +443,15 @@ __device__ __forceinline__ double ordered_sum_wave(const double* t, int n, doubl
             const int b0 = base + j * C;
 #pragma unroll
             for (int i = 0; i < C; ++i)
-                if (b0 + i < n) s = s + t[b0 + i];
+                if (b0 + i < n) s = s + get(b0 + i);
             base = b0 + C;
         }
     }
     return s;
+}
+template <int C>
+__device__ __forceinline__ double ordered_sum_wave(const double* t, int n, double s) {
+    return ordered_sum_wave_get<C>([t](int i) { return t[i]; }, n, s);
 }
 
 // Inclusive prefix sum over the lanes of one segment: lane l adds only the
@@ -475,203 +479,178 @@ __device__ __forceinline__ double wave_seg_scan_f64(double v, int ss, int lane) 
     return v;
 }
 
-// LDS of ordered_sum_block for W waves (records at the lane that ends a
-// segment).
+// LDS of ordered_sum_block for W waves.  A record is a segment or a
+// sequential lane; the first wave keeps up to kSumSlots0 of them, the others
+// kSumSlots, and the walk takes 64 in all.
+constexpr int kSumSlots0 = 32, kSumSlots = 8;
 template <int W>
 struct OrderedSumLds {
-    double wtot[W];               // plain sum of each wave's terms
-    unsigned long long items[W];  // lanes with a record: segment ends and sequential lanes
-    unsigned long long seql[W];   // the sequential lanes
-    double seg[W * 64];           // a segment's sum (incoming parity even), at its last lane
-    double flip[W * 64];          // its change for an odd incoming parity
-    int meta[W * 64];             // binade | first lane << 16
+    static constexpr int kSlots = kSumSlots0 + (W - 1) * kSumSlots;
+    double wtot[W];       // plain sum of each wave's terms
+    double even[kSlots];  // a segment's sum for an even incoming parity
+    double odd[kSlots];   // for an odd one
+    int seq[kSlots];      // a sequential lane's thread, or -1
+    int count[W];         // records of each wave
+    int list[64];         // the walk's records in order (slots)
     double result;
 };
 
 // Terms per lane of ordered_sum_block for n terms over 64W threads: the
-// smallest of 1, 3, 5, 11, 15, 17, 27, 33, 63 that covers n (odd, so the lanes'
-// blocks start in different LDS banks).  The term array must hold
-// 64 * W * ordered_sum_lane_terms(n, W) doubles; ordered_sum_block writes -0
-// past the n terms.
+// smallest of 3, 5, 11, 15, 27, 33 that covers n (odd, so the lanes' blocks
+// start in different LDS banks).
 __host__ __device__ constexpr int ordered_sum_lane_terms(int n, int w) {
     const int need = (n + 64 * w - 1) / (64 * w);
-    return need <= 1 ? 1 : need <= 3 ? 3 : need <= 5 ? 5 : need <= 11 ? 11 : need <= 15 ? 15
-         : need <= 17 ? 17 : need <= 27 ? 27 : need <= 33 ? 33 : 63;
-}
-__host__ __device__ constexpr int ordered_sum_slots(int n, int w) {
-    return 64 * w * ordered_sum_lane_terms(n, w);
+    return need <= 3 ? 3 : need <= 5 ? 5 : need <= 11 ? 11 : need <= 15 ? 15 : need <= 27 ? 27 : 33;
 }
 
-template <int W, int G>
-__device__ __forceinline__ double ordered_sum_block_g(double* t, int n, double s0,
-                                                     OrderedSumLds<W>& sh) {
-    constexpr int U = G < 8 ? G : (G <= 17 ? 8 : 4);  // reads in flight per lane
+// ordered_sum_block for G terms a lane, which get(i) (0 <= i < n) returns; every
+// thread of the workgroup calls it (waves past W only meet the barriers).
+template <int W, int G, typename Get>
+__device__ __forceinline__ double ordered_sum_core(Get get, int n, double s0, OrderedSumLds<W>& sh) {
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const bool active = wave < W;    // waves past W only meet the barriers
-    const double* tb = t + tid * G;  // this lane's block (active waves)
+    const bool active = wave < W;
 
-    // estimated running sums before and after each lane; an Inf or NaN term
-    // shows in the largest exponent field, a negative one in the smallest term
-    // (-0 padding is neither)
-    double a = 0.0, mn = 0.0, exc = 0.0;
-    unsigned hw = 0;
+    // this lane's terms (-0 past the n terms: s + -0 = s for every s), and the
+    // estimated running sums before and after them; a negative term shows in
+    // the smallest term (-0 padding is none), an Inf or NaN one in the sum
+    double t[G];
+    const auto term = [&](int i) {
+        const double v = get(min(i, n - 1));
+        return i < n ? v : -0.0;
+    };
+    double a = 0.0, exc = 0.0, mn = 0.0;
     if (active) {
-#pragma unroll(G <= 17 ? 8 : 1)
-    for (int i0 = 0; i0 < G; i0 += U) {
-        double v[U];
 #pragma unroll
-        for (int j = 0; j < U; ++j) v[j] = i0 + j < G ? tb[i0 + j] : 0.0;
+        for (int j = 0; j < G; ++j) t[j] = term(tid * G + j);
 #pragma unroll
-        for (int j = 0; j < U; ++j) {
-            if (i0 + j < G) {
-                a = a + v[j];
-                mn = fmin(mn, v[j]);
-                hw = max(hw, (unsigned)((unsigned long long)__double_as_longlong(v[j]) >> 32) & 0x7fffffffu);
-            }
+        for (int j = 0; j < G; ++j) {
+            a = a + t[j];
+            mn = fmin(mn, t[j]);
         }
-    }
-    const double inc = wave_scan_f64_dpp(a);
-    exc = __shfl_up(inc, 1, 64);
-    if (lane == 0) exc = 0.0;
-    if (lane == 63) sh.wtot[wave] = inc;
+        const double inc = wave_scan_f64_dpp(a);
+        exc = __shfl_up(inc, 1, 64);
+        if (lane == 0) exc = 0.0;
+        if (lane == 63) sh.wtot[wave] = inc;
     }
     __syncthreads();
+    int count = 0;
     if (active) {
-    double off = s0;
-#pragma unroll
-    for (int v = 0; v < W - 1; ++v) off = v < wave ? off + sh.wtot[v] : off;
-    const double lo = (off + exc) * (1.0 - 0x1p-30);
-    const double hi = ((off + exc) + a) * (1.0 + 0x1p-30);
-    int e = (int)((unsigned long long)__double_as_longlong(lo) >> 52);  // biased exponent
-    const bool sq = !(lo >= 0x1p-960 && hi < 0x1p1000 &&
-                      e == (int)((unsigned long long)__double_as_longlong(hi) >> 52) &&
-                      hw < 0x7ff00000u && mn >= 0.0);  // non-negative finite terms, one binade
-    if (sq) e = 1023;
-    const double scale = __longlong_as_double((long long)(2098 - e) << 52);  // 1/q
+        // the plain sum of the waves before this one (lane v of a 16-lane row
+        // takes wave v's, summed by DPP moves)
+        double off = lane < wave ? sh.wtot[min(lane, W - 1)] : 0.0;
+        off = off + dpp_rows_d<kDppShr1, 0xf>(off);
+        off = off + dpp_rows_d<kDppShr2, 0xf>(off);
+        off = off + dpp_rows_d<kDppShr4, 0xf>(off);
+        off = off + dpp_rows_d<kDppShr8, 0xf>(off);
+        off = s0 + readlane_d(off, 15);
+        const double lo = (off + exc) * (1.0 - 0x1p-30);
+        const double hi = ((off + exc) + a) * (1.0 + 0x1p-30);
+        int e = (int)((unsigned long long)__double_as_longlong(lo) >> 52);  // biased exponent
+        const bool sq = !(lo >= 0x1p-960 && hi < 0x1p1000 &&
+                          e == (int)((unsigned long long)__double_as_longlong(hi) >> 52));
+        const bool negative = __builtin_amdgcn_ballot_w64(!(mn >= 0.0)) != 0ull;
+        if (sq) e = 1023;
+        const double scale = __longlong_as_double((long long)(2098 - e) << 52);  // 1/q
+        const double q = __longlong_as_double((long long)(e - 52) << 52);
 
-    // this lane's terms in units of q, for an even incoming parity.  u + 2^52
-    // rounds u (0 <= u < 2^52 in a lane that keeps its binade) to the nearest
-    // integer, half even; at a half-integer an odd running sum takes the other
-    // neighbour u + (u - rn) instead.  The first tie changes the lane's sum by
-    // +-1 when the incoming parity is odd (flip).
-    double d0 = 0.0;
-    unsigned par = 0, tied = 0, flip = 0;
-#pragma unroll(G <= 17 ? 8 : 1)
-    for (int i0 = 0; i0 < G; i0 += U) {
-        double v[U];
+        // The chain itself from an even and from an odd running sum in units of
+        // q: 2^52 and 2^52 + 1 stand for them, since the lane's terms sum to
+        // less than 2^52 (a binade) and the last bit of every rounded sum in
+        // [2^52, 2^53) is its parity.  Until the first tie the two stay 1
+        // apart; from it on they are 0 or 2 apart, of one parity.
+        double c0 = 0x1p52, c1 = 0x1p52 + 1.0;
 #pragma unroll
-        for (int j = 0; j < U; ++j) v[j] = i0 + j < G ? tb[i0 + j] : 0.0;
-#pragma unroll
-        for (int j = 0; j < U; ++j) {
-            if (i0 + j < G) {
-                const double u = v[j] * scale;
-                const double w = u + 0x1p52;
-                const double rn = w - 0x1p52;
-                const double df = u - rn;  // exact
-                const unsigned odd = (unsigned)__double_as_longlong(w) & 1u;
-                const unsigned tie = fabs(df) == 0.5 ? 1u : 0u;
-                d0 = d0 + ((tie & par) ? u + df : rn);
-                const unsigned up = df > 0.0 ? 1u : 0u;
-                flip = (tie & ~tied) ? (up ^ par ^ 1u) : flip;  // 1: -1, 0: +1
-                tied |= tie;
-                par = tie ? 0u : (par ^ odd);
-            }
+        for (int j = 0; j < G; ++j) {
+            c0 = fma(t[j], scale, c0);  // (the product is exact)
+            c1 = fma(t[j], scale, c1);
         }
-    }
-    const double sgn = flip ? -1.0 : 1.0;
+        const double d0 = c0 - 0x1p52;
+        const double sgn = (c1 - c0) - 1.0;  // the change for an odd incoming parity
+        const bool tied = sgn != 0.0, par = (__double_as_longlong(c0) & 1ll) != 0;
 
-    // segments and each lane's incoming parity
-    const unsigned long long lt = (1ull << lane) - 1ull, le = lt | (1ull << lane);
-    const unsigned long long SQ = __builtin_amdgcn_ballot_w64(sq);
-    const int eprev = __shfl_up(e, 1, 64);
-    const bool start = !sq && (lane == 0 || ((SQ >> ((lane - 1) & 63)) & 1ull) || eprev != e);
-    const unsigned long long SS = __builtin_amdgcn_ballot_w64(start);
-    const unsigned long long ht = __builtin_amdgcn_ballot_w64(!sq && tied);
-    const unsigned long long po = __builtin_amdgcn_ballot_w64(!sq && tied && par);
-    const unsigned long long fp = __builtin_amdgcn_ballot_w64(!sq && !tied && par);
-    const int ss = sq ? lane + 1 : 63 - __builtin_clzll((SS & le) | 1ull);
-    const int ssc = sq ? lane : ss;
-    const unsigned long long inseg = lt & ~((1ull << ssc) - 1ull);  // segment lanes below
-    const unsigned long long below = ht & inseg;
-    const int b = below ? 63 - __builtin_clzll(below) : -1;       // last tie below
-    const unsigned long long since = b >= 0 ? (lt & ~((2ull << b) - 1ull)) : inseg;
-    const int p0 = b >= 0 ? (int)((po >> b) & 1ull) : 0;
-    const int pin = p0 ^ (__builtin_popcountll(fp & since) & 1);
-    const double d = sq ? 0.0 : ((tied && pin) ? d0 + sgn : d0);
-    const double dl = (!sq && tied && b < 0) ? (pin ? -sgn : sgn) : 0.0;
-    const double psum = wave_seg_scan_f64(d, ss, lane);
-    const bool end = !sq && (lane == 63 || (((SS | SQ) >> ((lane + 1) & 63)) & 1ull));
-    const unsigned long long SE = __builtin_amdgcn_ballot_w64(end);
-    const unsigned long long ft = ht & ~((1ull << ssc) - 1ull) & le;  // ties from the segment start
-    const double fl = __shfl(dl, ft ? __builtin_ctzll(ft) : lane, 64);
-    if (end) {
-        sh.seg[tid] = psum;
-        sh.flip[tid] = ft ? fl : 0.0;
-        sh.meta[tid] = e | (ss << 16);
-    }
-    if (lane == 0) {
-        sh.items[wave] = SE | SQ;
-        sh.seql[wave] = SQ;
-    }
+        // segments and each lane's incoming parity
+        const unsigned long long lt = (1ull << lane) - 1ull, le = lt | (1ull << lane);
+        const unsigned long long SQ = __builtin_amdgcn_ballot_w64(sq);
+        const int eprev = __shfl_up(e, 1, 64);
+        const bool start = !sq && (lane == 0 || ((SQ >> ((lane - 1) & 63)) & 1ull) || eprev != e);
+        const unsigned long long SS = __builtin_amdgcn_ballot_w64(start);
+        const unsigned long long ht = __builtin_amdgcn_ballot_w64(!sq && tied);
+        const unsigned long long po = __builtin_amdgcn_ballot_w64(!sq && tied && par);
+        const unsigned long long fp = __builtin_amdgcn_ballot_w64(!sq && !tied && par);
+        const int ss = sq ? lane + 1 : 63 - __builtin_clzll((SS & le) | 1ull);
+        const int ssc = sq ? lane : ss;
+        const unsigned long long inseg = lt & ~((1ull << ssc) - 1ull);  // segment lanes below
+        const unsigned long long below = ht & inseg;
+        const int b = below ? 63 - __builtin_clzll(below) : -1;       // last tie below
+        const unsigned long long since = b >= 0 ? (lt & ~((2ull << b) - 1ull)) : inseg;
+        const int p0 = b >= 0 ? (int)((po >> b) & 1ull) : 0;
+        const int pin = p0 ^ (__builtin_popcountll(fp & since) & 1);
+        const double d = sq ? 0.0 : (pin ? d0 + sgn : d0);
+        const int dl = (!sq && tied && b < 0) ? (pin ? -(int)sgn : (int)sgn) : 0;
+        const double psum = wave_seg_scan_f64(d, ss, lane);
+        const bool end = !sq && (lane == 63 || (((SS | SQ) >> ((lane + 1) & 63)) & 1ull));
+        const unsigned long long items = __builtin_amdgcn_ballot_w64(end || sq);
+        const unsigned long long ft = ht & ~((1ull << ssc) - 1ull) & le;  // ties from the segment start
+        const int fl = __shfl(dl, ft ? __builtin_ctzll(ft) : lane, 64);
+        const int slots = wave == 0 ? kSumSlots0 : kSumSlots;
+        const int at = __builtin_popcountll(items & lt);
+        if ((end || sq) && at < slots) {
+            const int sl = (wave == 0 ? 0 : kSumSlots0 + (wave - 1) * kSumSlots) + at;
+            sh.even[sl] = psum * q;  // as it is added: an integer times q, exact
+            sh.odd[sl] = (ft ? psum + (double)fl : psum) * q;
+            sh.seq[sl] = sq ? tid : -1;
+        }
+        count = __builtin_popcountll(items);
+        if (negative || count > slots) count = 1 << 16;  // (the walk gives up)
+        if (lane == 0) sh.count[wave] = count;
     }
     __syncthreads();
 
-    // wave 0 walks the records in order (a failed check ends the walk and
-    // the remaining terms go through ordered_sum_wave); the next wave's records
-    // are read while the current wave's are walked
+    // Wave 0 walks the records in order, one a lane.  Every record is a chain
+    // of G additions to the running sum: a sequential lane's terms, or a
+    // segment's sum for the running sum's parity (the last bit of its
+    // significand) and G - 1 times -0, so a step has no branch: every lane
+    // adds its own record to the running sum and the record's lane is taken.
     if (wave == 0) {
+        // lane w lists wave w's records behind those of the waves before it
+        const int own = lane < W ? sh.count[min(lane, W - 1)] : 0;
+        int upto = own;
+        upto += dpp_i<kDppShr1>(upto, 0);
+        upto += dpp_i<kDppShr2>(upto, 0);
+        upto += dpp_i<kDppShr4>(upto, 0);
+        upto += dpp_i<kDppShr8>(upto, 0);
+        const int N = __builtin_amdgcn_readlane(upto, 15);
         double s = s0;
-        int rest = -1;
-        double segv = sh.seg[lane], flipv = sh.flip[lane];
-        int metav = sh.meta[lane];
-        unsigned long long itv = sh.items[0], sqv = sh.seql[0];
-        for (int w = 0; w < W && rest < 0; ++w) {
-            unsigned long long items = uniform_u64(itv);
-            const unsigned long long seqm = uniform_u64(sqv);
-            const double cseg = segv, cflip = flipv;
-            const int cmeta = metav;
-            if (w + 1 < W) {
-                segv = sh.seg[(w + 1) * 64 + lane];
-                flipv = sh.flip[(w + 1) * 64 + lane];
-                metav = sh.meta[(w + 1) * 64 + lane];
-                itv = sh.items[w + 1];
-                sqv = sh.seql[w + 1];
-            }
-            while (items) {
-                const int l = __builtin_ctzll(items);
-                items &= items - 1ull;
-                const int b0 = (w * 64 + l) * G;
-                if ((seqm >> l) & 1ull) {
-                    // a sequential lane: its G terms, read U ahead of the additions
-                    // (the padding past n is -0, and s + -0 = s for every s)
-                    const double* sb = t + b0;
-#pragma unroll(G <= 17 ? 8 : 1)
-                    for (int i0 = 0; i0 < G; i0 += U) {
-                        double v[U];
+        if (N <= 64) {
+            if (lane < count) sh.list[lane] = lane;  // wave 0's own
 #pragma unroll
-                        for (int j = 0; j < U; ++j) v[j] = i0 + j < G ? sb[i0 + j] : 0.0;
+            for (int i = 0; i < kSumSlots; ++i)
+                if (lane > 0 && i < own) sh.list[upto - own + i] = kSumSlots0 + (lane - 1) * kSumSlots + i;
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // the list is written
+            __builtin_amdgcn_wave_barrier();
+            const int sl = lane < N ? sh.list[lane] : 0;
+            const int sq = lane < N ? sh.seq[sl] : -1;
+            double ev = lane < N ? sh.even[sl] : -0.0, od = lane < N ? sh.odd[sl] : -0.0;
+            const int base = sq >= 0 ? sq * G : n;  // (terms past n are -0)
 #pragma unroll
-                        for (int j = 0; j < U; ++j)
-                            if (i0 + j < G) s = s + v[j];
-                    }
-                    continue;
+            for (int j = 0; j < G; ++j) t[j] = term(base + j);
+            if (sq >= 0) ev = od = t[0];
+            const long long eb = __double_as_longlong(ev), ob = __double_as_longlong(od);
+            for (int r0 = 0; r0 < N; r0 += 4) {  // (lanes past N add -0)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int mask = -(__double2loint(s) & 1);
+                    const int lo = ((int)ob & mask) | ((int)eb & ~mask);
+                    const int hi = ((int)(ob >> 32) & mask) | ((int)(eb >> 32) & ~mask);
+                    double x = s + __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+#pragma unroll
+                    for (int j = 1; j < G; ++j) x = x + t[j];
+                    s = readlane_d(x, r0 + i);
                 }
-                const int meta = __builtin_amdgcn_readlane(cmeta, l);
-                const int E = meta & 0x7ff;
-                const double sc = __longlong_as_double((long long)(2098 - E) << 52);
-                const double q = __longlong_as_double((long long)(E - 52) << 52);
-                const double seg = readlane_d(cseg, l), fv = readlane_d(cflip, l);
-                const double su = s * sc;
-                const double D = seg + ((__double_as_longlong(su) & 1ll) ? fv : 0.0);
-                const bool ok = (int)((unsigned long long)__double_as_longlong(s) >> 52) == E && D < 0x1p53 - su;
-                if (__builtin_expect(!ok, 0)) {
-                    rest = (w * 64 + (meta >> 16)) * G;
-                    break;
-                }
-                s = (su + D) * q;
             }
+        } else {
+            s = ordered_sum_wave_get<kChainC>(get, n, s0);
         }
-        if (rest >= 0) s = ordered_sum_wave<kChainC>(t + rest, n - rest, s);
         if (lane == 0) sh.result = s;
     }
     __syncthreads();
@@ -680,10 +659,8 @@ __device__ __forceinline__ double ordered_sum_block_g(double* t, int n, double s
 
 // The one-lane chain `for (i = 0; i < n; ++i) s = s + t[i];` (t in LDS), bit
 // for bit, formed by the first W waves of the workgroup (every thread of the
-// workgroup calls it -- waves past W only meet its four barriers -- and every
-// thread gets the result).  t must
-// hold ordered_sum_slots(n, W) doubles: the slots past n are set to -0, which
-// leaves every sum unchanged.
+// workgroup calls it after a barrier that follows the writes of t -- waves past
+// W only meet its three barriers -- and every thread gets the result).
 //
 // Thread g takes the G = ordered_sum_lane_terms(n, W) consecutive terms
 // [gG, gG + G).  A plain fp64 prefix sum of the lanes' totals estimates the
@@ -691,47 +668,43 @@ __device__ __forceinline__ double ordered_sum_block_g(double* t, int n, double s
 // non-negative terms), which places each lane in the binade [2^E, 2^(E+1))
 // its running sum keeps throughout -- with a margin of 2^-30 either side --
 // or marks it sequential (a crossing of a power of two, a zero or tiny start,
-// a huge end, a negative or non-finite term).  In a binade every rounded sum
-// is a multiple of q = 2^(E-52) and s + t rounds to s + q * r with r = t/q
-// rounded to the nearest integer, except at a half-integer t/q, whose
-// round-half-even result is the candidate that leaves s/q even (see
-// ordered_sum_wave).  So a lane sums its r in units of q exactly, taking its
-// segment's incoming parity as even; a run of lanes with one binade forms a
-// segment whose sum is a segmented prefix sum over the lanes (exact: integers
-// below 2^53), where each lane's parity comes from wave ballots, and whose sum
-// for an odd incoming parity differs only at its first tie.  Wave 0 then walks
-// the records in order: a segment checks that the exact running sum lies in
-// its binade with room for the segment's sum and adds it (its parity picks the
-// variant); a sequential lane adds its terms with fp64 additions.  A failed
-// check (a running sum the estimate misplaced: possible only with negative
-// terms) hands the rest of the row, from that segment's first term, to
-// ordered_sum_wave.
+// a huge or non-finite end).  In a binade every rounded sum is a multiple of
+// q = 2^(E-52), and s + t rounds to s + q * r with r = t/q rounded to the
+// nearest integer, except at a half-integer t/q, whose round-half-even result
+// is the candidate that leaves s/q even: what a lane adds depends on the
+// running sum through its parity alone.  So a lane forms its chain for both
+// parities (two fused multiply-adds a term); a run of lanes with one binade
+// forms a segment whose sum is a segmented prefix sum over the lanes (exact:
+// integers below 2^52), where each lane's parity comes from wave ballots, and
+// whose sum for an odd incoming parity differs only at its first tie.  Wave 0
+// then walks the records in order: a segment adds its sum (the running sum's
+// parity picks the variant), a sequential lane its terms.  A row with a
+// negative term (the estimate bounds non-negative ones only), or with more
+// records than the slots, goes through ordered_sum_wave.
+//
+// What bounds it is latency.  Stamps of the cycle counter on gfx950 (6,912
+// squares of normal values, eight waves, 24 records): the terms and their plain
+// sums 1,350 cycles, the two chains and the segments 1,950, gathering the
+// records 1,450, the walk 3,900.  A walk that looped over the records with a
+// branch per kind took 7,100 (about 220 cycles a record beside its additions,
+// 7.5 cycles each), one with the checks in fp64 9,900; sixteen waves of half
+// the terms walk 34 records in 4,170 cycles and wait longer for each other.
 template <int W>
-__device__ __forceinline__ double ordered_sum_block(double* t, int n, double s0,
+__device__ __forceinline__ double ordered_sum_block(const double* t, int n, double s0,
                                                    OrderedSumLds<W>& sh) {
-    static_assert(W >= 2 && W <= 8, "the sum runs on 2 to 8 waves");
+    static_assert(W == 4 || W == 8, "the sum runs on four or eight waves");
     if (n <= 0) return s0;
+    const auto get = [t](int i) { return t[i]; };
     const int G = ordered_sum_lane_terms(n, W);
-    for (int i = n + (int)threadIdx.x; i < 64 * W * G; i += (int)blockDim.x) t[i] = -0.0;
-    __syncthreads();
-    switch (G) {
-        case 1: return ordered_sum_block_g<W, 1>(t, n, s0, sh);
-        case 3: return ordered_sum_block_g<W, 3>(t, n, s0, sh);
-        case 5: return ordered_sum_block_g<W, 5>(t, n, s0, sh);
-        case 11: return ordered_sum_block_g<W, 11>(t, n, s0, sh);
-        case 15: return ordered_sum_block_g<W, 15>(t, n, s0, sh);
-        case 17: return ordered_sum_block_g<W, 17>(t, n, s0, sh);
-        default: break;
+    constexpr int kMax = ordered_sum_lane_terms(kMaxStrictNormCols, W);
+    if (G == 3) return ordered_sum_core<W, 3>(get, n, s0, sh);
+    if (G == 5) return ordered_sum_core<W, 5>(get, n, s0, sh);
+    if (G == 11) return ordered_sum_core<W, 11>(get, n, s0, sh);
+    if (G == 15) return ordered_sum_core<W, 15>(get, n, s0, sh);
+    if constexpr (kMax > 27) {
+        if (G == 27) return ordered_sum_core<W, 27>(get, n, s0, sh);
     }
-    if constexpr (W <= 4) {  // more than 17 terms per lane (n <= 8064) only below 8 waves
-        switch (G) {
-            case 27: return ordered_sum_block_g<W, 27>(t, n, s0, sh);
-            case 33: return ordered_sum_block_g<W, 33>(t, n, s0, sh);
-            default: break;
-        }
-    }
-    if constexpr (W <= 2) return ordered_sum_block_g<W, 63>(t, n, s0, sh);
-    return ordered_sum_wave<kChainC>(t, n, s0);  // (not reached for n <= 8064)
+    return ordered_sum_core<W, kMax>(get, n, s0, sh);
 }
 
 // Block reductions over blockDim.x threads (a multiple of 64, at most 1024).

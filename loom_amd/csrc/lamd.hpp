@@ -167,6 +167,9 @@ struct RowNormArgs {
 // rows or outputs not 16-byte aligned, n beyond the kernel's register budget,
 // strict without totals, or LOOM_AMD_ROWNORM_WAVE=0.
 bool launch_row_norm_wave(int kind, int strict, const RowNormArgs& a, hipStream_t s, hipError_t* e);
+// The same with one workgroup of eight or sixteen waves per row (any number of
+// rows); strict mode forms the ordered sums itself.
+bool launch_row_norm_block(int kind, int strict, const RowNormArgs& a, hipStream_t s, hipError_t* e);
 
 // Strict ordered sums of squares of m fp32 rows (one lane per row, in element
 // order) into totals when m is large enough and the rows are 16-byte aligned;

@@ -1478,12 +1478,10 @@ constexpr int kNormWaves = 8;
 constexpr int kNormThreads = kNormWaves * 64;
 
 // Dynamic LDS of a norm-fused launch: the quantized rows, or in strict mode
-// the row's squares padded for ordered_sum_block (four waves, or eight for
-// rows of kSumWideCols and more).
+// the row's squares.
 static size_t norm_lds(int m, int k, int strict) {
     const size_t q = (size_t)m * pad_cols(k);
-    const int slots = max(ordered_sum_slots(k, 4), k >= kSumWideCols ? ordered_sum_slots(k, 8) : 0);
-    const size_t sq = strict ? (size_t)slots * 8 : 0;
+    const size_t sq = strict ? (size_t)k * 8 : 0;
     return q > sq ? q : sq;
 }
 

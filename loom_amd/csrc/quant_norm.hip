@@ -605,6 +605,251 @@ bool launch_row_norm_wave(int kind, int strict, const RowNormArgs& a, hipStream_
     return true;
 }
 
+// ------------------------------------------------------------------------
+// Row norm + requantization, one workgroup of W waves per row (fewer rows than
+// the one-wave kernel wants: decode batches to mid-size prompts).  Thread t
+// holds the four-column groups t and t + 64 W (16-byte loads, the four codes
+// of a group as one 32-bit store), so a thread normalizes and rounds at most
+// eight values; with 256 threads and one column every 256 it was 27 of 6,912.
+// What bounds it is latency: one load round trip, the sum, one division and
+// one exchange for the maximum.  Inner norm of 8 rows on gfx950, one launch in
+// a graph: 6,912 columns strict 22.5 -> 8.1 us, fast 9.4 -> 5.1; 2,560 columns
+// 11.4 -> 6.3 and 5.4 -> 3.8 (256 rows: 23.7 -> 9.6, 10.5 -> 6.6, 11.9 -> 6.9,
+// 5.9 -> 4.4).
+//   fast: the row's values go through LDS and thread c of 256 sums columns c,
+//     c + 256, ... in order, then the pairs (t, t + w) for w = 128, ..., 1:
+//     the tree of the other row-norm kernels, so the same bits.
+//   strict: ordered_sum_core on eight waves (G consecutive columns a thread).
+// The fp32 rounding of the division by the rms is decided as in the norm-fused
+// GEMVs: p = (v y) g with y = 1 / rms lies within 5 * 2^-53 |p| of loom's fp64
+// value, so if p -+ |p| 2^-50 round to one float that float is loom's result;
+// a group with an undecided value divides.
+// ------------------------------------------------------------------------
+
+constexpr int kRowBlockWide = 4096;  // columns: eight waves up to here, sixteen above (two groups a thread)
+
+template <int KIND, int STRICT, int W, int G>
+__global__ __launch_bounds__(W * 64) void row_norm_block_kernel(RowNormArgs a) {
+    using T = typename std::conditional<KIND == kRowInnerF64, double, float>::type;
+    constexpr bool F64 = KIND == kRowInnerF64;
+    constexpr int NT = W * 64, NG = 2;
+    extern __shared__ __align__(16) char dynsh[];  // the row's n values
+    T* vals = (T*)dynsh;
+    __shared__ typename std::conditional<STRICT != 0, OrderedSumLds<8>, double[256]>::type sums;
+    __shared__ unsigned shm[W];
+    __shared__ int shs[W];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int row = blockIdx.x, n = a.n, n4 = n >> 2;
+    const T* xr = (const T*)a.x + (size_t)row * a.ldx;
+    T v[NG][4];
+    float4 w4[NG];
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+        const int g = tid + NT * j, c = 4 * min(g, n4 - 1);
+        if constexpr (F64) {
+            const double2 p0 = *(const double2*)(xr + c), p1 = *(const double2*)(xr + c + 2);
+            v[j][0] = p0.x, v[j][1] = p0.y, v[j][2] = p1.x, v[j][3] = p1.y;
+        } else {
+            const float4 p0 = *(const float4*)(xr + c);
+            v[j][0] = p0.x, v[j][1] = p0.y, v[j][2] = p0.z, v[j][3] = p0.w;
+        }
+        w4[j] = a.w ? *(const float4*)(a.w + c) : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+    }
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+        const int g = tid + NT * j;
+        if (g < n4) {
+            if constexpr (F64) {
+                *(double2*)(vals + 4 * g) = make_double2(v[j][0], v[j][1]);
+                *(double2*)(vals + 4 * g + 2) = make_double2(v[j][2], v[j][3]);
+            } else {
+                *(float4*)(vals + 4 * g) = make_float4(v[j][0], v[j][1], v[j][2], v[j][3]);
+            }
+        }
+    }
+    __syncthreads();
+    double total;
+    if constexpr (STRICT != 0) {
+        total = ordered_sum_core<8, G>([vals](int i) { const double f = (double)vals[i]; return f * f; }, n, 0.0, sums);
+    } else {
+        if (tid < 256) {
+            double p = 0.0;
+#pragma unroll 4
+            for (int c = tid; c < n; c += 256) {
+                const double f = (double)vals[c];
+                p = p + f * f;
+            }
+            sums[tid] = p;
+        }
+        __syncthreads();
+        double t = (sums[lane] + sums[lane + 128]) + (sums[lane + 64] + sums[lane + 192]);
+#pragma unroll
+        for (int w = 32; w > 0; w >>= 1) t = t + __shfl_down(t, w, 64);
+        total = __shfl(t, 0, 64);
+    }
+
+    const double ms = total / (double)n + a.eps;
+    unsigned lb = 0u;  // largest |value| bit pattern (fp32 rows); F64: of its fp32 rounding
+    if constexpr (KIND == kRowRms) {
+        const double rms = sqrt(ms), y = 1.0 / rms;
+#pragma unroll
+        for (int j = 0; j < NG; ++j) {
+            const float gf[4] = {w4[j].x, w4[j].y, w4[j].z, w4[j].w};
+            float o[4];
+            bool redo = false;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const double p = ((double)v[j][i] * y) * (double)gf[i];
+                const double d = fabs(p) * 0x1p-50;
+                o[i] = (float)(p - d);
+                redo |= !(o[i] == (float)(p + d));
+            }
+            if (redo) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = (float)(((double)v[j][i] / rms) * (double)gf[i]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[j][i] = o[i];
+        }
+    } else {
+        const double scale = 1.0 / sqrt(ms);
+#pragma unroll
+        for (int j = 0; j < NG; ++j) {
+            const double g[4] = {w4[j].x, w4[j].y, w4[j].z, w4[j].w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (F64)
+                    v[j][i] = v[j][i] * (scale * g[i]);
+                else
+                    v[j][i] = (float)((double)v[j][i] * scale * g[i]);
+            }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+        const int g = tid + NT * j;
+        if (g >= n4) continue;
+        const int c = 4 * g;
+        if constexpr (F64) {
+            if (a.keep64) {
+                double* kr = a.keep64 + (size_t)row * a.ldx + c;
+                *(double2*)kr = make_double2(v[j][0], v[j][1]);
+                *(double2*)(kr + 2) = make_double2(v[j][2], v[j][3]);
+            }
+            if (a.yf)
+                *(float4*)(a.yf + (size_t)row * n + c) =
+                    make_float4((float)v[j][0], (float)v[j][1], (float)v[j][2], (float)v[j][3]);
+        } else if (a.yf) {
+            *(float4*)(a.yf + (size_t)row * (KIND == kRowRms ? (long)n : a.ldx) + c) =
+                make_float4(v[j][0], v[j][1], v[j][2], v[j][3]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) lb = max(lb, __float_as_uint(fabsf((float)v[j][i])));
+    }
+    lb = wave_umax_dpp(lb);
+    if (lane == 0) shm[wave] = lb;
+    __syncthreads();
+    unsigned mb = shm[0];
+#pragma unroll
+    for (int w = 1; w < W; ++w) mb = max(mb, shm[w]);
+    const bool gen = mb > 0x7f7fffffu;  // NaN or infinity in the row (uniform)
+    float m = __uint_as_float(mb);
+    if (gen) {  // loom's NaN-skipping maximum
+        float lm = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NG; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (tid + NT * j < n4) lm = max_nan_skip(lm, fabsf((float)v[j][i]));
+        lm = wave_max_dpp(lm);
+        __syncthreads();  // (every thread has read shm)
+        if (lane == 0) shm[wave] = __float_as_uint(lm);
+        __syncthreads();
+        m = 0.0f;
+#pragma unroll
+        for (int w = 0; w < W; ++w) m = max_nan_skip(m, __uint_as_float(shm[w]));
+    }
+    if (m < 1e-5f) m = 1e-5f;
+    if (!a.xq) return;  // (uniform: the normalized rows only)
+    const double qs = 127.0 / (double)m;
+    const float qs32 = (float)qs;
+    const float sf = F64 || gen ? 0.0f : 127.0f / m;  // (as act_quant_rows_kernel)
+    int sum = 0;
+    uint32_t* qr = (uint32_t*)(a.xq + (size_t)row * a.ldq);
+#pragma unroll
+    for (int j = 0; j < NG; ++j) {
+        const int g = tid + NT * j;
+        if (g >= n4) continue;
+        uint32_t pk;
+        if constexpr (F64) {
+            pk = pack4(quant_one(v[j][0], qs), quant_one(v[j][1], qs), quant_one(v[j][2], qs), quant_one(v[j][3], qs));
+        } else {
+            const float p0 = v[j][0] * sf, p1 = v[j][1] * sf, p2 = v[j][2] * sf, p3 = v[j][3] * sf;
+            const float r0 = rintf(p0), r1 = rintf(p1), r2 = rintf(p2), r3 = rintf(p3);
+            const float d = fmaxf(fmaxf(fabsf(p0 - r0), fabsf(p1 - r1)), fmaxf(fabsf(p2 - r2), fabsf(p3 - r3)));
+            pk = pack4((int)r0, (int)r1, (int)r2, (int)r3);
+            if (gen || !(0.5f - d > 3.1e-5f))
+                pk = pack4(quant_f32(v[j][0], qs32, qs), quant_f32(v[j][1], qs32, qs), quant_f32(v[j][2], qs32, qs),
+                           quant_f32(v[j][3], qs32, qs));
+        }
+        qr[g] = pk;
+        sum = byte_sum_i8(pk, sum);
+    }
+    for (int g = n4 + tid; g < (a.ldq >> 2); g += NT) qr[g] = 0u;  // padding columns
+    sum = wave_sum_i(sum);
+    if (lane == 0) shs[wave] = sum;
+    __syncthreads();
+    if (tid == 0) {
+        int t = 0;
+#pragma unroll
+        for (int w = 0; w < W; ++w) t += shs[w];
+        a.amax[row] = m;
+        a.xsum[row] = t;
+    }
+}
+
+// Launches the W-wave kernel and returns true, or returns false (nothing
+// launched) when the rows do not qualify: n % 4 != 0, rows or outputs not
+// 16-byte aligned, totals already formed, or LOOM_AMD_ROWNORM_BLOCK=0.
+bool launch_row_norm_block(int kind, int strict, const RowNormArgs& a, hipStream_t s, hipError_t* e) {
+    if (tune_int("LOOM_AMD_ROWNORM_BLOCK", 1) == 0 || a.totals) return false;
+    if (a.m <= 0 || a.n <= 0 || a.n % 4 != 0 || a.n > kMaxNormCols || (strict && a.n > kMaxStrictNormCols)) return false;
+    if (a.xq && (a.ldq % 4 != 0 || a.ldq < a.n || ((uintptr_t)a.xq & 3) != 0)) return false;
+    const size_t es = kind == kRowInnerF64 ? 8 : 4;
+    auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+    if (!al16(a.x) || ((size_t)a.ldx * es) % 16 != 0 || !al16(a.w) || !al16(a.yf) || !al16(a.keep64)) return false;
+    const size_t shm = (size_t)a.n * es;
+    const bool wide = a.n > kRowBlockWide;
+    const int g = ceil_div(a.n, 512);  // terms per lane of the ordered sum
+#define LAMD_RNB(K, S, W, G) \
+    hipLaunchKernelGGL((row_norm_block_kernel<K, S, W, G>), dim3(a.m), dim3(64 * W), shm, s, a)
+#define LAMD_RNB_KIND(K)                             \
+    do {                                             \
+        if (!strict) {                               \
+            if (wide) LAMD_RNB(K, 0, 16, 1);         \
+            else LAMD_RNB(K, 0, 8, 1);               \
+        } else if (wide) {                           \
+            if (g <= 11) LAMD_RNB(K, 1, 16, 11);     \
+            else if (g <= 15) LAMD_RNB(K, 1, 16, 15);\
+            else LAMD_RNB(K, 1, 16, 17);             \
+        } else {                                     \
+            if (g <= 3) LAMD_RNB(K, 1, 8, 3);        \
+            else if (g <= 5) LAMD_RNB(K, 1, 8, 5);   \
+            else LAMD_RNB(K, 1, 8, 9);               \
+        }                                            \
+    } while (0)
+    if (kind == kRowRms)
+        LAMD_RNB_KIND(kRowRms);
+    else if (kind == kRowInner)
+        LAMD_RNB_KIND(kRowInner);
+    else
+        LAMD_RNB_KIND(kRowInnerF64);
+#undef LAMD_RNB_KIND
+#undef LAMD_RNB
+    *e = hipGetLastError();
+    return true;
+}
+
 template <int STRICT>
 static hipError_t launch_norm_t(float* h, int ldh, int m, int n, const float* weight, double eps,
                                 int8_t* hq, int ldq, float* amax, int32_t* xsum, int keep,
@@ -613,8 +858,9 @@ static hipError_t launch_norm_t(float* h, int ldh, int m, int n, const float* we
         const RowNormArgs a{h, ldh, m, n, weight, eps, keep ? h : nullptr, nullptr, hq, ldq, amax, xsum, totals};
         hipError_t e = hipSuccess;
         if (launch_row_norm_wave(kRowInner, STRICT, a, s, &e)) return e;
+        if (launch_row_norm_block(kRowInner, STRICT, a, s, &e)) return e;
     }
-    const size_t shm = STRICT && !totals ? (size_t)ordered_sum_slots(n, 4) * sizeof(double)
+    const size_t shm = STRICT && !totals ? (size_t)n * sizeof(double)
                                          : 256 * sizeof(double);
     const dim3 g(m), b(256);
 #define LAMD_NQ(VPT)                                                                            \
@@ -648,9 +894,8 @@ hipError_t launch_norm_quant(float* h, int ldh, int m, int n, const float* weigh
 }
 
 // One workgroup per row: the row's n terms into LDS, then the index-order
-// chain s0 + t[0] + t[1] + ... formed by ordered_sum_wave (64 threads) or
-// ordered_sum_block on four waves (256 or 512 threads: the strict norm
-// kernels' widths).
+// chain s0 + t[0] + t[1] + ... formed by ordered_sum_wave (W = 1) or
+// ordered_sum_block on W waves: the widths of the strict norm kernels.
 template <int W>
 __global__ __launch_bounds__(W * 64) void ordered_sum_rows_kernel(const double* __restrict__ terms, int n,
                                                                   double s0, double* __restrict__ out) {
@@ -661,27 +906,31 @@ __global__ __launch_bounds__(W * 64) void ordered_sum_rows_kernel(const double* 
     double r;
     if constexpr (W == 1) {
         r = ordered_sum_wave<kChainC>(tsh, n, s0);
-    } else {  // the first four waves form the sum
-        __shared__ OrderedSumLds<4> osum;
-        r = ordered_sum_block<4>(tsh, n, s0, osum);
+    } else {
+        __shared__ OrderedSumLds<W> osum;
+        r = ordered_sum_block<W>(tsh, n, s0, osum);
     }
     if (threadIdx.x == 0) out[blockIdx.x] = r;
 }
 
+// threads = 64, 256 or 512: one, four or eight waves.
 hipError_t launch_ordered_sum_rows(const double* terms, int m, int n, double s0, double* out,
                                    int threads, hipStream_t s) {
     if (m <= 0) return hipSuccess;
     if (n <= 0 || n > kMaxStrictNormCols) return hipErrorInvalidValue;
-    const size_t shm = (size_t)max(n, ordered_sum_slots(n, threads < 256 ? 1 : 4)) * sizeof(double);
+    const size_t shm = (size_t)n * sizeof(double);
+#define LAMD_OSR(W) \
+    hipLaunchKernelGGL(ordered_sum_rows_kernel<W>, dim3(m), dim3(64 * W), shm, s, terms, n, s0, out)
     if (threads == 64) {
-        hipLaunchKernelGGL(ordered_sum_rows_kernel<1>, dim3(m), dim3(64), shm, s, terms, n, s0, out);
+        LAMD_OSR(1);
     } else if (threads == 256) {
-        hipLaunchKernelGGL(ordered_sum_rows_kernel<4>, dim3(m), dim3(256), shm, s, terms, n, s0, out);
+        LAMD_OSR(4);
     } else if (threads == 512) {
-        hipLaunchKernelGGL(ordered_sum_rows_kernel<8>, dim3(m), dim3(512), shm, s, terms, n, s0, out);
+        LAMD_OSR(8);
     } else {
         return hipErrorInvalidValue;
     }
+#undef LAMD_OSR
     return hipGetLastError();
 }
 

@@ -933,3 +933,26 @@ def test_lm_head_rows_equal_single_rows(torch_dev, tf, sequential, rows, vocab, 
         one = tf.lm_head(table, x[r:r + 1].clone(), sequential)[0]
         assert torch.equal(got[r].isnan(), one.isnan()), r
         assert torch.equal(got[r].nan_to_num(0.5), one.nan_to_num(0.5)), r
+
+
+@pytest.mark.parametrize("norm", ["strict", "fast"])
+@pytest.mark.parametrize("hidden,heads,inter,seq", [(2560, 20, 6912, 40), (256, 4, 516, 5)])
+def test_block_row_norm_workgroups_agree(orc, torch_dev, tf, tuning, norm, hidden, heads, inter, seq):
+    # RMSNorm, the fp64 MHA inner norm and the SwiGLU inner norm on eight- and
+    # sixteen-wave workgroups: every tap is the bytes of the 256-thread kernels
+    # (LOOM_AMD_ROWNORM_BLOCK=0)
+    torch = torch_dev
+    sh = Shape(hidden, heads, heads, hidden // heads, inter, 64)
+    w = Weights(orc, sh, seed=1501, act=ACT_SILU)
+    gw = w.gpu(tf)
+    x_in = orc.normal_f32(seq * hidden, 1502).reshape(seq, hidden)
+    outs = {}
+    for block in (1, 0):
+        tuning("LOOM_AMD_ROWNORM_BLOCK", block)
+        blk = tf.BitNetBlock(w.cfg(tf, norm), gw)
+        x = to_dev(torch, x_in)
+        _, t = blk.forward(x, taps=True)
+        torch.cuda.synchronize()
+        outs[block] = [x.cpu().numpy().tobytes()] + [a.tobytes() for a in t.numpy().values()]
+        blk.release()
+    assert outs[1] == outs[0]

@@ -162,3 +162,33 @@ def test_ordered_sum_rows_rejects_bad_shapes(torch_dev):
     assert lib.loom_amd_ordered_sum_rows(None, 1, 4, C.c_double(0.0), o, 256, None) == -1
     assert lib.loom_amd_ordered_sum_rows(p, 1, 4, C.c_double(0.0), o, 128, None) == -1
     assert lib.loom_amd_ordered_sum_rows(p, 0, 4, C.c_double(0.0), o, 256, None) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("norm", ["strict", "fast"])
+@pytest.mark.parametrize("n", [4, 252, 1536, 1540, 2560, 4092, 4096, 4100, 5636, 6912, 7684, 8064])
+def test_row_norm_workgroups_agree(torch_dev, tuning, norm, n):
+    # the eight- and sixteen-wave row norms give the bytes of the 256-thread
+    # kernels: terms-per-lane steps of the ordered sum, both workgroup widths,
+    # zero, huge, tiny, leading-zero, outlier, NaN and Inf rows
+    torch = torch_dev
+    from loom_amd import bitnet as bn
+    rng = np.random.default_rng(n)
+    h = rng.standard_normal((12, n)).astype(np.float32)
+    h[1] = 0.0
+    h[2] *= np.float32(1e18)
+    h[3] *= np.float32(1e-20)
+    h[4, : n - 1] = 0.0
+    h[5, rng.integers(0, n, 6)] *= np.float32(4096.0)
+    h[6, n // 2] = np.nan
+    h[7, n // 3] = np.inf
+    h[8] = np.float32(0.5) * rng.integers(-3, 4, n)
+    h[9] *= np.exp(rng.uniform(-20, 20, n)).astype(np.float32)
+    w = torch.from_numpy(rng.uniform(0.5, 1.5, n).astype(np.float32)).cuda()
+    got = {}
+    for block in (1, 0):
+        tuning("LOOM_AMD_ROWNORM_BLOCK", block)
+        x = torch.from_numpy(h).cuda()
+        q = bn.norm_quant_rows(x, w, 1e-5, norm)
+        got[block] = [t.cpu().numpy().tobytes() for t in (x, q.xq, q.amax, q.xsum)]
+    assert got[1] == got[0]

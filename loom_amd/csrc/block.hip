@@ -2036,33 +2036,42 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const int* __restrict
 // strict part 2: one workgroup per (head, group of DG value columns, row).
 // The probabilities p[k] = exp(score[k] - max) are formed here: the maximum
 // over the chunk maxima (every wave forms it), then one probability per thread
-// and 256-position chunk into an LDS ring two chunks deep.  Lane d <= DG of
+// and 256 positions into an LDS ring two chunks deep.  Lane d <= DG of
 // wave 0 adds column d of the products p[k] * v[k][d] in position order (the
 // reference's `sum += p * v`, a product then a sum, each rounded); column DG
-// holds p itself, whose chain is expSum.  Chunks of C = 4096 / DG positions:
-// each of the 256 threads of waves 1-4 loads its 16 values of a chunk (and
-// the scores it turns into probabilities: C / 256) kChainDepth chunks ahead,
-// forms its products in registers and writes them to one of two LDS product
-// buffers, transposed so that a chain lane reads two positions per 16-byte
-// load; wave 0 only adds: chunk c while the other waves write the products of
-// chunk c + 1 and the probabilities of chunk c + 2.  The loads are
-// branch-free (indices clamped into the ring and the score row; surplus
-// values are never added).  grid (heads * HD / DG, rows), 320 threads.
+// holds p itself, whose chain is expSum.  Chunks of C positions: each of the
+// 256 threads of waves 1-4 loads its C DG / 256 values of a chunk (and the
+// scores it turns into probabilities) kChainDepth chunks ahead, forms its
+// products in registers and writes them to one of two LDS product buffers,
+// transposed so that a chain lane reads two positions per 16-byte load; wave 0
+// only adds: chunk c while the other waves write the products of chunk c + 1
+// and the probabilities of chunk c + 2.  The loads are branch-free (indices
+// clamped into the ring and the score row); products past the last position
+// are -0, which leaves a sum as it is, so wave 0 adds whole groups of 32.
+// What bounds it: for one row the chains (7.5 cycles an addition), for several
+// the rounds of workgroups.  One row takes DG = 16, C = 256 (74 KB of LDS, two
+// workgroups a CU), more rows DG = 32, C = 64 (36 KB, four a CU), so eight rows
+// of 20 heads are one round instead of two and a half.  A strict decode layer
+// at BitNet-2B shape (gfx950, us; the head's share included): one row at 2,048
+// positions 98.5 with a branch in every sixteen additions and barriers that
+// wait for the loads, 87.3 now (90.2 with DG = 32); two rows 92.4 with DG = 32,
+// 106.3 with DG = 16; eight rows at 120 positions 86 -> 82, at 2,048 151 -> 130.
+// grid (heads * HD / DG, rows), 320 threads.
 constexpr int kChainDepth = 4;
-constexpr int kChainCols = 16;
+constexpr int kChainWideRows = 2;
 constexpr int kChainThreads = 320;  // wave 0: the chains; waves 1-4: loads, probabilities, products
 
-template <int HD, int DG>
+template <int HD, int DG, int C>
 __global__ __launch_bounds__(kChainThreads) void attn_chain_kernel(const float* __restrict__ cache_v,
                                                          const int* __restrict__ pos0, int msl,
                                                          int span, int heads, int kv_heads,
                                                          int seq, DecodeScratch sc,
                                                          double* __restrict__ out) {
-    constexpr int C = 4096 / DG;  // positions per chunk
-    constexpr int CP = C + 2;     // row pitch (16-byte aligned rows, lanes' reads in different banks)
-    static_assert(C * DG == 4096 && C % 256 == 0 && C <= 512 && HD % DG == 0 && DG % 4 == 0,
+    constexpr int NV = C * DG / 1024;  // 16-byte loads per thread and chunk
+    constexpr int CP = C + 2;          // row pitch (16-byte aligned rows, lanes' reads in different banks)
+    static_assert(NV * 1024 == C * DG && (NV == 2 || NV == 4) && C % 64 == 0 && C <= 256 && HD % DG == 0 &&
+                      DG % 4 == 0 && DG < 64,
                   "chunk geometry");
-    constexpr int PT = C / 256;   // probabilities per thread and chunk
     __shared__ __align__(16) double prod[2][DG + 1][CP];
     __shared__ double pr_sh[2][C];
     const int h = blockIdx.x / (HD / DG), dg = blockIdx.x % (HD / DG), row = blockIdx.y;
@@ -2085,14 +2094,14 @@ __global__ __launch_bounds__(kChainThreads) void attn_chain_kernel(const float* 
 
     // staging registers of the chunks in flight (named scalars filled by
     // macros: arrays of them, indexed in loops, were kept in scratch memory).
-    // Thread tid holds the float4s at elements 4(tid + 256 I) of the chunk's
-    // C x DG values (position e / DG, column e % DG) and the scores of
-    // positions tid + 256 q.
+    // Thread pt holds the float4s at elements 4(pt + 256 I) of the chunk's
+    // C x DG values (position e / DG, column e % DG) and the score of position
+    // pt (threads past C: of no position).
     float4 r0_0, r0_1, r0_2, r0_3, r1_0, r1_1, r1_2, r1_3;
     float4 r2_0, r2_1, r2_2, r2_3, r3_0, r3_1, r3_2, r3_3;
-    double pt0[PT], pt1[PT], pt2[PT], pt3[PT];
+    double pt0, pt1, pt2, pt3;
 #define LAMD_CHAIN_LD(U, I, CC)                                                   \
-    {                                                                             \
+    if ((I) < NV) {                                                               \
         const int e = (pt + (I) * 256) * 4; /* element of the C x DG chunk */     \
         const int k = (CC) * C + e / DG;                                          \
         r##U##_##I = *(const float4*)(vb + (size_t)min(k, msl - 1) * kv_dim + e % DG); \
@@ -2102,94 +2111,90 @@ __global__ __launch_bounds__(kChainThreads) void attn_chain_kernel(const float* 
         const int cc = min((CH), nch - 1);                                        \
         LAMD_CHAIN_LD(U, 0, cc) LAMD_CHAIN_LD(U, 1, cc)                           \
         LAMD_CHAIN_LD(U, 2, cc) LAMD_CHAIN_LD(U, 3, cc)                           \
-        _Pragma("unroll") for (int q = 0; q < PT; ++q)                            \
-            pt##U[q] = sr[min(cc * C + pt + 256 * q, span - 1)];                 \
+        pt##U = sr[min(cc * C + min(pt, C - 1), span - 1)];                       \
     }
 #define LAMD_CHAIN_EXP(U, BUF)                                                    \
     {                                                                             \
-        _Pragma("unroll") for (int q = 0; q < PT; ++q)                            \
-            pr_sh[BUF][pt + 256 * q] = exp(pt##U[q] - mx);                       \
+        const double p = exp(pt##U - mx);                                         \
+        if (pt < C) pr_sh[BUF][pt] = p;                                           \
     }
-#define LAMD_CHAIN_PR(U, I, BUF)                                                  \
-    {                                                                             \
+#define LAMD_CHAIN_PR(U, I, BUF, CC)                                              \
+    if ((I) < NV) {                                                               \
         const int e = (pt + (I) * 256) * 4;                                      \
         const int k = e / DG, d = e % DG;                                         \
         const double p = pr_sh[BUF][k];                                           \
-        prod[BUF][d][k] = p * (double)r##U##_##I.x;                               \
-        prod[BUF][d + 1][k] = p * (double)r##U##_##I.y;                           \
-        prod[BUF][d + 2][k] = p * (double)r##U##_##I.z;                           \
-        prod[BUF][d + 3][k] = p * (double)r##U##_##I.w;                           \
+        const bool in = (CC) * C + k < L;                                         \
+        prod[BUF][d][k] = in ? p * (double)r##U##_##I.x : -0.0;                   \
+        prod[BUF][d + 1][k] = in ? p * (double)r##U##_##I.y : -0.0;               \
+        prod[BUF][d + 2][k] = in ? p * (double)r##U##_##I.z : -0.0;               \
+        prod[BUF][d + 3][k] = in ? p * (double)r##U##_##I.w : -0.0;               \
     }
-#define LAMD_CHAIN_PRODUCTS(U, BUF)                                               \
+#define LAMD_CHAIN_PRODUCTS(U, BUF, CC)                                           \
     {                                                                             \
-        LAMD_CHAIN_PR(U, 0, BUF) LAMD_CHAIN_PR(U, 1, BUF)                         \
-        LAMD_CHAIN_PR(U, 2, BUF) LAMD_CHAIN_PR(U, 3, BUF)                         \
-        _Pragma("unroll") for (int q = 0; q < PT; ++q)                            \
-            prod[BUF][DG][pt + 256 * q] = pr_sh[BUF][pt + 256 * q];             \
+        LAMD_CHAIN_PR(U, 0, BUF, CC) LAMD_CHAIN_PR(U, 1, BUF, CC)                 \
+        LAMD_CHAIN_PR(U, 2, BUF, CC) LAMD_CHAIN_PR(U, 3, BUF, CC)                 \
+        if (pt < C) prod[BUF][DG][pt] = (CC) * C + pt < L ? pr_sh[BUF][pt] : -0.0; \
     }
+    // The two roles run separate loops (one's registers are free in the
+    // other's) that meet at the same barriers: two before the first chunk, one
+    // after each.  The barriers wait for LDS only, so the loads of the next
+    // chunks stay in flight across them.
+    double sum = 0.0;  // column tid's chain (tid <= DG)
     if (maker) {
         LAMD_CHAIN_ISSUE(0, 0)
         LAMD_CHAIN_ISSUE(1, 1)
         LAMD_CHAIN_ISSUE(2, 2)
         LAMD_CHAIN_ISSUE(3, 3)
-    }
-    // maximum over the chunk maxima of the 64-position score chunks with
-    // data: -1e9 start, NaN never wins (each wave forms the same value)
-    double mx = -1e9;
-    {
-        const double* cm = sc.cmax + rh * attn_nchunk(span);
-        const int nc = (L + 63) / 64;
-        for (int c = lane; c < nc; c += 64) {
-            const double v = cm[c];
-            mx = v > mx ? v : mx;
+        // maximum over the chunk maxima of the 64-position score chunks with
+        // data: -1e9 start, NaN never wins (each wave forms the same value)
+        double mx = -1e9;
+        {
+            const double* cm = sc.cmax + rh * attn_nchunk(span);
+            const int nc = (L + 63) / 64;
+            for (int c = lane; c < nc; c += 64) {
+                const double v = cm[c];
+                mx = v > mx ? v : mx;
+            }
+            for (int off = 32; off > 0; off >>= 1) {
+                const double o = __shfl_xor(mx, off, 64);
+                mx = o > mx ? o : mx;
+            }
         }
-        for (int off = 32; off > 0; off >>= 1) {
-            const double o = __shfl_xor(mx, off, 64);
-            mx = o > mx ? o : mx;
-        }
-    }
-    if (maker) {
         LAMD_CHAIN_EXP(0, 0)
         LAMD_CHAIN_EXP(1, 1)
-    }
-    __syncthreads();
-    if (maker) {
-        LAMD_CHAIN_PRODUCTS(0, 0)
+        tile_lds_barrier();
+        LAMD_CHAIN_PRODUCTS(0, 0, 0)
         LAMD_CHAIN_ISSUE(0, kChainDepth)
-    }
-    __syncthreads();
-
-    double sum = 0.0;  // column tid's chain (tid <= DG)
-    // step for chunk c = c0 + U: waves 1-4 write the products of chunk c + 1
-    // (staging set U + 1) to buffer (c + 1) & 1 and refill that set, and the
-    // probabilities of chunk c + 2 (set UE) to ring slot c & 1, while wave 0
-    // adds chunk c from buffer c & 1 (all parities are compile-time: c0 is a
-    // multiple of four).  Products, probabilities and loads run for every
-    // chunk's step, for chunks past the last one too (clamped indices; no
-    // chain reads them), so the loads of the next three chunks stay in flight
-    // across each wait.
+        tile_lds_barrier();
+        // step for chunk c = c0 + U: the products of chunk c + 1 (staging set
+        // U + 1) to buffer (c + 1) & 1, that set's refill, and the
+        // probabilities of chunk c + 2 (set UE) to ring slot c & 1, while wave
+        // 0 adds chunk c from buffer c & 1 (all parities are compile-time: c0
+        // is a multiple of four).  They run for chunks past the last one too
+        // (clamped indices; no chain reads them).
 #define LAMD_CHAIN_STEP(U, UN, UE)                                                \
     {                                                                             \
         const int c = c0 + (U);                                                   \
         if (c >= nch) break;                                                      \
-        if (maker) {                                                               \
-            LAMD_CHAIN_PRODUCTS(UN, ((U) + 1) & 1)                                \
-            LAMD_CHAIN_EXP(UE, (U) & 1)                                           \
-            LAMD_CHAIN_ISSUE(UN, c + 1 + kChainDepth)                             \
-        }                                                                         \
-        if (c < nch && tid <= DG) {                                               \
-            const double* pc = prod[(U) & 1][tid];                                \
-            const int n = min(C, L - c * C);                                      \
-            sum = chain_add_pairs<C>(pc, n, sum);                                 \
-        }                                                                         \
-        __syncthreads();                                                          \
+        LAMD_CHAIN_PRODUCTS(UN, ((U) + 1) & 1, c + 1)                             \
+        LAMD_CHAIN_EXP(UE, (U) & 1)                                               \
+        LAMD_CHAIN_ISSUE(UN, c + 1 + kChainDepth)                                 \
+        tile_lds_barrier();                                                            \
     }
-    static_assert(kChainDepth == 4, "the loop below expands four chunk steps");
-    for (int c0 = 0; c0 < nch; c0 += kChainDepth) {
-        LAMD_CHAIN_STEP(0, 1, 2)
-        LAMD_CHAIN_STEP(1, 2, 3)
-        LAMD_CHAIN_STEP(2, 3, 0)
-        LAMD_CHAIN_STEP(3, 0, 1)
+        static_assert(kChainDepth == 4, "the loop below expands four chunk steps");
+        for (int c0 = 0; c0 < nch; c0 += kChainDepth) {
+            LAMD_CHAIN_STEP(0, 1, 2)
+            LAMD_CHAIN_STEP(1, 2, 3)
+            LAMD_CHAIN_STEP(2, 3, 0)
+            LAMD_CHAIN_STEP(3, 0, 1)
+        }
+    } else {
+        tile_lds_barrier();
+        tile_lds_barrier();
+        for (int c = 0; c < nch; ++c) {
+            if (tid <= DG) sum = chain_add_groups(prod[c & 1][tid], (min(C, L - c * C) + 31) >> 5, sum);
+            tile_lds_barrier();
+        }
     }
 #undef LAMD_CHAIN_STEP
 #undef LAMD_CHAIN_PRODUCTS
@@ -2255,7 +2260,7 @@ static hipError_t launch_strict_decode(const double* q, float* cache_k, float* c
                                        const RopeArgs& ra, double* out, hipStream_t s) {
     const int nc = attn_nchunk(span);
     const dim3 gs(kv_heads, nc, rows), t(256);
-    constexpr int DG = kChainCols;
+    const bool wide = rows >= kChainWideRows;
 #define LAMD_SCORES(HDV)                                                                          \
     {                                                                                             \
         if (ra.acc && (ra.qk.q || ra.qk.k))                                                       \
@@ -2268,9 +2273,13 @@ static hipError_t launch_strict_decode(const double* q, float* cache_k, float* c
             hipLaunchKernelGGL((attn_scores_gqa_kernel<HDV, false>), gs, t, 0, s, q, cache_k,       \
                                cache_v, pos0, msl, span, heads, kv_heads, seq, sc, ra);           \
     }
-#define LAMD_CHAIN(HDV)                                                                              \
-    hipLaunchKernelGGL((attn_chain_kernel<HDV, DG>), dim3(heads * (HDV / DG), rows), dim3(kChainThreads), 0, \
-                       s, cache_v, pos0, msl, span, heads, kv_heads, seq, sc, out)
+#define LAMD_CHAIN(HDV)                                                                                      \
+    if (wide)                                                                                                \
+        hipLaunchKernelGGL((attn_chain_kernel<HDV, 32, 64>), dim3(heads * (HDV / 32), rows), dim3(kChainThreads), \
+                           0, s, cache_v, pos0, msl, span, heads, kv_heads, seq, sc, out);                  \
+    else                                                                                                     \
+        hipLaunchKernelGGL((attn_chain_kernel<HDV, 16, 256>), dim3(heads * (HDV / 16), rows),              \
+                           dim3(kChainThreads), 0, s, cache_v, pos0, msl, span, heads, kv_heads, seq, sc, out)
     switch (hd) {
         case 32: LAMD_SCORES(32); break;
         case 64: LAMD_SCORES(64); break;
@@ -2840,8 +2849,7 @@ __global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restri
         for (int k = 0; k < kHeadAhead; ++k) load_w(32 * k, ring[k], std::false_type{});
     }
     store_x(xs[0]);
-    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
-    __builtin_amdgcn_s_barrier();
+    tile_lds_barrier();
     for (int i = 0; i < nslab; ++i) {
         const int c0 = i * kHeadCols;
         const float* buf = xs[i & 1];
@@ -2854,8 +2862,7 @@ __global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restri
             load_w(cn + 32 * k, ring[k], std::false_type{});
         }
         store_x(xs[(i & 1) ^ 1]);  // last read before the previous barrier
-        __builtin_amdgcn_s_waitcnt(0xc07f);
-        __builtin_amdgcn_s_barrier();
+        tile_lds_barrier();
     }
     for (int k = 0; k < nrest; ++k) {
         uint32_t w[8];

@@ -787,11 +787,19 @@ void loom_amd_model_release(loom_amd_model* m) {
     if (m) free_model(m);
 }
 
-// Rows that the screened greedy head takes one after another (about 78 us a
-// row at vocab 128256 x 2560, 38 us at 32000); above, the full head of all
-// rows in one pass over the table is shorter (302 us and 76 us for 2 to 16
-// rows, sequential order 655 us).
-constexpr int kScreenMaxRows = 3;
+// Whether a greedy head of `batch` rows screens them one after another (the
+// int8 codes once a row) or forms every logit in one pass over the fp32 table.
+// Measured in us on gfx950 (hidden 2560; x = entries over those of vocab
+// 128256): a screened row 28 + 50 x (three short launches and the codes), the
+// full head of 2 to 16 rows and its pick 20 + 302 x (655 x in sequential
+// order), of one row 20 + 195 x and more than the screened row for every table
+// that a model has.
+static bool head_screens(const loom_amd_model* m, int batch) {
+    if (!m->lm_q || tune_int("LOOM_AMD_LM_SCREEN", 1) == 0) return false;
+    if (batch == 1) return true;
+    const double x = (double)m->vocab * m->hidden / (128256.0 * 2560.0);
+    return batch * (28.0 + 50.0 * x) <= 20.0 + (m->lm_sequential ? 655.0 : 302.0) * x * ceil_div(batch, 16);
+}
 
 // Final norm + LM head + argmax of each sequence's last row (row stride ld
 // floats between sequences), writing the token at *pos + offset.
@@ -832,7 +840,7 @@ static int model_head(loom_amd_model* m, const float* last, long ld, int batch, 
             }
         }
         if (e != hipSuccess) return fail_hip("model ternary lm head", e);
-    } else if (m->lm_q && batch <= kScreenMaxRows && tune_int("LOOM_AMD_LM_SCREEN", 1) != 0) {
+    } else if (head_screens(m, batch)) {
         // greedy pick from an int8 screening pass and the candidates' exact
         // logits, one row after the other (the bounds and the threshold are
         // per row; every call leaves the threshold cleared)

@@ -266,45 +266,40 @@ __device__ __forceinline__ unsigned wave_umax_dpp(unsigned v) {
     return (unsigned)__builtin_amdgcn_readlane(b, 63);
 }
 
-// s + p[base] + ... + p[base + 15] in index order, the terms past n replaced
-// by -0 (s + -0 = s for every s).
-__device__ __forceinline__ double add_block16(const double2 (&v)[8], int base, int n, double s) {
-    if (base + 16 <= n) {
+// s + p[0] + p[1] + ... in index order over `groups` >= 1 groups of 32 terms (one
+// lane; p in LDS, 16-byte aligned), two terms per 16-byte read, the next group
+// read while one is added.  One branch in 64 terms: a branch costs as much as
+// six additions here, and with one or two in every 16 terms a chain took 20
+// cycles a term instead of about 9.
+__device__ __forceinline__ double chain_add_groups(const double* p, int groups, double s) {
+    const double2* p2 = (const double2*)p;
+    double2 a[16], b[16];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            s = s + v[j].x;
-            s = s + v[j].y;
+    for (int j = 0; j < 16; ++j) a[j] = p2[j];
+    int g = 0;
+#pragma clang loop unroll(disable)
+    for (; g + 2 <= groups; g += 2) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) b[j] = p2[(g + 1) * 16 + j];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            s = s + a[j].x;
+            s = s + a[j].y;
         }
-    } else {
+        const int next = min(g + 2, groups - 1);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            s = s + (base + 2 * j < n ? v[j].x : -0.0);
-            s = s + (base + 2 * j + 1 < n ? v[j].y : -0.0);
+        for (int j = 0; j < 16; ++j) a[j] = p2[next * 16 + j];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            s = s + b[j].x;
+            s = s + b[j].y;
         }
     }
-    return s;
-}
-
-// s + p[0] + p[1] + ... + p[n-1] in index order (one lane; p in LDS, 16-byte
-// aligned, C doubles readable, n <= C), two terms per 16-byte read, with the
-// reads of four blocks of sixteen terms in flight ahead of the additions
-// (reads past n are never added).
-template <int C>
-__device__ __forceinline__ double chain_add_pairs(const double* p, int n, double s) {
-    static_assert(C % 16 == 0, "blocks of sixteen terms");
-    const double2* p2 = (const double2*)p;
-    constexpr int NB = C / 16, D = NB < 4 ? NB : 4;
-    double2 v[D][8];
+    if (g < groups) {
 #pragma unroll
-    for (int b = 0; b < D; ++b)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[b][j] = p2[b * 8 + j];
-#pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        if (b * 16 < n) s = add_block16(v[b % D], b * 16, n, s);
-        if (b + D < NB) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[b % D][j] = p2[(b + D) * 8 + j];
+        for (int j = 0; j < 16; ++j) {
+            s = s + a[j].x;
+            s = s + a[j].y;
         }
     }
     return s;

@@ -956,3 +956,30 @@ def test_block_row_norm_workgroups_agree(orc, torch_dev, tf, tuning, norm, hidde
         outs[block] = [x.cpu().numpy().tobytes()] + [a.tobytes() for a in t.numpy().values()]
         blk.release()
     assert outs[1] == outs[0]
+
+
+@pytest.mark.parametrize("hd", [32, 128])
+@pytest.mark.parametrize("prompt", [2, 30, 62, 126, 254, 318])
+def test_strict_decode_chains_at_chunk_edges(orc, torch_dev, tf, hd, prompt):
+    # the strict decode chains of several rows (64-position chunks) give the
+    # bits of the one-row form (256-position chunks), stepping over the edges of
+    # chunks and of the 32-term groups that a partial chunk is added in
+    torch = torch_dev
+    heads = 4
+    sh = Shape(256, heads, 2, hd, 512, 336)
+    w = Weights(orc, sh, seed=1601, act=ACT_SILU)
+    gw = w.gpu(tf)
+    cfg = w.cfg(tf, "strict")
+    cfg.max_batch = 2
+    both, one = tf.BitNetBlock(cfg, gw), tf.BitNetBlock(cfg, gw)
+    x = orc.normal_f32(2 * prompt * sh.hidden, 1602 + prompt).reshape(2, prompt, sh.hidden)
+    steps = orc.normal_f32(2 * 4 * sh.hidden, 1603).reshape(4, 2, 1, sh.hidden)
+    both.forward(to_dev(torch, x))
+    got = [both.forward(to_dev(torch, s))[0].cpu().numpy() for s in steps]
+    for b in range(2):
+        one.forward(to_dev(torch, x[b:b + 1]))
+        for s, g in zip(steps, got):
+            r = one.forward(to_dev(torch, s[b:b + 1]))[0].cpu().numpy()
+            assert g[b].tobytes() == r[0].tobytes()
+    both.release()
+    one.release()

@@ -594,7 +594,7 @@ int loom_amd_swiglu_forward(const loom_amd_matrix* gate, const loom_amd_matrix* 
     gu.ldo = inter;
     gu.acc0 = taps ? taps->acc_gate : nullptr;
     gu.acc1 = taps ? taps->acc_up : nullptr;
-    const bool fused = fused_quant_ok(m, hidden, x);
+    const bool fused = fused_quant_ok(m, hidden, x, true);
     hipError_t e;
     if (fused) {
         e = launch_matmul_fused(&G, &U, x, m, gu, taps ? taps->xq : nullptr,

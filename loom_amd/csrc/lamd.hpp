@@ -98,7 +98,7 @@ hipError_t launch_matmul(const Matrix* w0, const Matrix* w1, const QuantAct& a, 
 // Same, quantizing fp32 rows x (M x K, row stride K) inside the matmul kernel
 // (one launch).  Only for the shapes fused_quant_ok accepts.  xq_tap (M x K)
 // and amax_tap (M) optionally receive the quantized rows.
-bool fused_quant_ok(int m, int k, const float* x);
+bool fused_quant_ok(int m, int k, const float* x, bool two = false);
 hipError_t launch_matmul_fused(const Matrix* w0, const Matrix* w1, const float* x, int m,
                                const Epilogue& epi, int8_t* xq_tap, float* amax_tap,
                                hipStream_t s);

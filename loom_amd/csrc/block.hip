@@ -740,6 +740,52 @@ __device__ __forceinline__ void tile_pv_whole(const double* __restrict__ pr, con
     }
 }
 
+// PV over a chunk that some queries of the tile see in part: query i of the
+// lane's four takes positions kk <= lim + i (and the lane's expSum query those
+// <= es_lim), the others are computed and not taken (selects, no branch: a loop
+// to each query's own end waited for its LDS reads position by position, about
+// 11 us a tile at head size 128 against 2).
+template <int HD>
+__device__ __forceinline__ void tile_pv_masked(const double* __restrict__ pr, const double* __restrict__ pe,
+                                               const double* __restrict__ vr, int lim, int es_lim,
+                                               double (&acc)[4][HD / 32], double& es) {
+    constexpr int DB = HD / 32;
+    constexpr int PP = kChunkP + 2;
+#pragma unroll 2
+    for (int kk = 0; kk < kChunkP; kk += 2) {
+        double2 pk[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) pk[i] = *(const double2*)(pr + i * PP + kk);
+        const double2 e = *(const double2*)(pe + kk);
+        const double e0 = es + e.x;
+        es = kk <= es_lim ? e0 : es;
+        const double e1 = es + e.y;
+        es = kk + 1 <= es_lim ? e1 : es;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            double v[DB];
+            const double2 va = *(const double2*)(vr + (kk + u) * HD);
+            v[0] = va.x;
+            v[1] = va.y;
+            if constexpr (DB == 4) {
+                const double2 vc = *(const double2*)(vr + (kk + u) * HD + 64);
+                v[2] = vc.x;
+                v[3] = vc.y;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const double pv = u ? pk[i].y : pk[i].x;
+                const bool in = kk + u <= lim + i;
+#pragma unroll
+                for (int j = 0; j < DB; ++j) {
+                    const double t = acc[i][j] + pv * v[j];
+                    acc[i][j] = in ? t : acc[i][j];
+                }
+            }
+        }
+    }
+}
+
 template <int HD>
 __global__ __launch_bounds__(256) void attn_tile_kernel(const double* __restrict__ q,
                                                         const float* __restrict__ cache_k,
@@ -905,33 +951,7 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(const double* __restrict
             else
                 tile_pv_whole<HD, false>(&sm.p[4 * pq * PP], pe, vr, acc, es);
         } else {
-            if (tid < kTileQ) {
-                const int lim = base + s0 + tid;
-                for (int kk = 0; kk < kChunkP; kk += 2) {
-                    const double2 pk = *(const double2*)(pe + kk);
-                    if (kc + kk <= lim) es += pk.x;
-                    if (kc + kk + 1 <= lim) es += pk.y;
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int qi = 4 * pq + i;
-                const int n = min(kChunkP, base + s0 + qi + 1 - kc);  // valid positions of this chunk
-                for (int kk = 0; kk < n; ++kk) {
-                    const double pk = sm.p[qi * PP + kk];
-                    double v[DB];
-                    const double2 va = *(const double2*)(vr + kk * HD);
-                    v[0] = va.x;
-                    v[1] = va.y;
-                    if constexpr (DB == 4) {
-                        const double2 vc = *(const double2*)(vr + kk * HD + 64);
-                        v[2] = vc.x;
-                        v[3] = vc.y;
-                    }
-#pragma unroll
-                    for (int j = 0; j < DB; ++j) acc[i][j] = acc[i][j] + pk * v[j];
-                }
-            }
+            tile_pv_masked<HD>(&sm.p[4 * pq * PP], pe, vr, base + s0 + 4 * pq - kc, base + s0 + tid - kc, acc, es);
         }
         tile_lds_barrier();  // chunk c's reads done before chunk c + 1 is staged
     }
@@ -946,6 +966,242 @@ __global__ __launch_bounds__(256) void attn_tile_kernel(const double* __restrict
 #pragma unroll
             for (int j = 0; j < DB; ++j)
                 out[(row0 + qi) * q_dim + (size_t)h * HD + 64 * (j >> 1) + 2 * dl + (j & 1)] = acc[i][j] / e;
+        }
+    }
+}
+
+// Strict prefill attention of few tiles, in two launches.  attn_tile_kernel
+// gives a tile one workgroup for both passes, so a prompt whose tiles do not
+// fill the chip waits for its longest tile: at 512 positions and 20 heads 320
+// workgroups, the last tiles' 16 chunks twice over 157 us while the work of all
+// is 38 us of the chip.  Here the score pass is cut by positions (scores and a
+// maximum do not depend on their order): kScoreParts workgroups a tile, each a
+// range of its chunks, write the scores and the range's maxima; and the value
+// pass is cut by columns (each column's chain runs over all positions): one
+// workgroup per 64 columns forms the tile's probabilities and chains again.
+// Same expressions and orders as attn_tile_kernel, so the same bits.  At 512
+// positions 57 + 59 us, near the fp64 issue of the passes (the probabilities
+// are formed twice) and the staging of three rounds of score workgroups.
+constexpr int kScoreParts = 4;
+
+template <int HD>
+__global__ __launch_bounds__(256) void attn_tile_scores_kernel(const double* __restrict__ q,
+                                                               const float* __restrict__ cache_k,
+                                                               const int* __restrict__ pos0, int msl, int span,
+                                                               int heads, int kv_heads, int seq,
+                                                               double* __restrict__ sc_all,
+                                                               double* __restrict__ pmax) {
+    using Lds = TileLds<HD>;
+    constexpr int QP = Lds::QP, KP = Lds::KP;
+    constexpr int F4 = kChunkP * HD / 4 / 256;  // float4 per thread per chunk
+    __shared__ __align__(16) double sq[kTileQ * QP];
+    __shared__ __align__(16) double sk[kChunkP * KP];
+    const int tid = threadIdx.x;
+    const int h = blockIdx.x;
+    const int tile = gridDim.y - 1 - blockIdx.y;  // longest tiles first
+    const int b = blockIdx.z / kScoreParts, part = blockIdx.z % kScoreParts;
+    const int s0 = tile * kTileQ;
+    const int nq = min(kTileQ, seq - s0);
+    const int base = *pos0;
+    const int q_dim = heads * HD, kv_dim = kv_heads * HD;
+    const int kvh = h / (heads / kv_heads);
+    const size_t row0 = (size_t)b * seq + s0;
+    if (base + s0 + nq > span) return;  // (the value pass writes NaN)
+    const int nch = (base + s0 + nq + kChunkP - 1) / kChunkP;
+    const int c0 = nch * part / kScoreParts, c1 = nch * (part + 1) / kScoreParts;
+    const float* kb = cache_k + (size_t)b * msl * kv_dim + (size_t)kvh * HD;
+    const int qp = tid >> 4, pp = tid & 15;
+    const int qa = 2 * qp;
+    const int lim_a = base + s0 + qa;  // last position query qa sees
+    const double scale = 1.0 / sqrt((double)HD);
+    const bool w0 = qa < nq, w1 = qa + 1 < nq;
+    double* sca = sc_all + ((row0 + min(qa, nq - 1)) * heads + h) * (size_t)span;
+    const size_t sc_next = w1 ? (size_t)heads * span : 0;  // row qa+1
+    double m0 = -1e9, m1 = -1e9;
+    if (c0 < c1) {  // (workgroup-uniform)
+        float4 rk[F4];
+        auto load = [&](int c) {
+#pragma unroll
+            for (int j = 0; j < F4; ++j) {
+                const int e = (tid + j * 256) * 4;
+                rk[j] = *(const float4*)(kb + (size_t)min(c * kChunkP + e / HD, msl - 1) * kv_dim + e % HD);
+            }
+        };
+        load(c0);
+        for (int i = tid; i < kTileQ * HD; i += 256) {
+            const int qi = i / HD;
+            sq[qi * QP + i % HD] = qi < nq ? q[(row0 + qi) * q_dim + (size_t)h * HD + i % HD] : 0.0;
+        }
+        for (int c = c0; c < c1; ++c) {
+#pragma unroll
+            for (int j = 0; j < F4; ++j) {  // K chunk: k[position][d]
+                const int e = (tid + j * 256) * 4;
+                double* d = &sk[(e / HD) * KP + e % HD];
+                *(double2*)d = make_double2((double)rk[j].x, (double)rk[j].y);
+                *(double2*)(d + 2) = make_double2((double)rk[j].z, (double)rk[j].w);
+            }
+            load(min(c + 1, c1 - 1));  // prefetch
+            tile_lds_barrier();        // chunk c (and the Q rows) staged
+            double d00 = 0.0, d01 = 0.0, d10 = 0.0, d11 = 0.0;
+            const double* q0 = &sq[qa * QP];
+            const double* q1 = q0 + QP;
+            const double* k0 = &sk[pp * KP];
+            const double* k1 = k0 + 16 * KP;
+#pragma unroll 8
+            for (int d = 0; d < HD; d += 2) {
+                const double2 a0 = *(const double2*)(q0 + d), a1 = *(const double2*)(q1 + d);
+                const double2 b0 = *(const double2*)(k0 + d), b1 = *(const double2*)(k1 + d);
+                d00 += a0.x * b0.x;
+                d01 += a0.x * b1.x;
+                d10 += a1.x * b0.x;
+                d11 += a1.x * b1.x;
+                d00 += a0.y * b0.y;
+                d01 += a0.y * b1.y;
+                d10 += a1.y * b0.y;
+                d11 += a1.y * b1.y;
+            }
+            const double s00 = d00 * scale, s01 = d01 * scale, s10 = d10 * scale, s11 = d11 * scale;
+            const int k = c * kChunkP + pp;  // positions k and k + 16
+            if (k < span) {
+                if (w0) sca[k] = s00;
+                if (w1) sca[sc_next + k] = s10;
+            }
+            if (k + 16 < span) {
+                if (w0) sca[k + 16] = s01;
+                if (w1) sca[sc_next + k + 16] = s11;
+            }
+            if (k <= lim_a && s00 > m0) m0 = s00;
+            if (k + 16 <= lim_a && s01 > m0) m0 = s01;
+            if (k <= lim_a + 1 && s10 > m1) m1 = s10;
+            if (k + 16 <= lim_a + 1 && s11 > m1) m1 = s11;
+            tile_lds_barrier();  // chunk c read before chunk c + 1 overwrites it
+        }
+        // maximum over the 16 lanes of each query pair (order-free)
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) {
+            const double o0 = __shfl_xor(m0, off, 16), o1 = __shfl_xor(m1, off, 16);
+            m0 = o0 > m0 ? o0 : m0;
+            m1 = o1 > m1 ? o1 : m1;
+        }
+    }
+    if (pp == 0) {
+        if (w0) pmax[((row0 + qa) * heads + h) * kScoreParts + part] = m0;
+        if (w1) pmax[((row0 + qa + 1) * heads + h) * kScoreParts + part] = m1;
+    }
+}
+
+template <int HD>
+__global__ __launch_bounds__(256) void attn_tile_values_kernel(const float* __restrict__ cache_v,
+                                                               const int* __restrict__ pos0, int msl, int span,
+                                                               int heads, int kv_heads, int seq,
+                                                               const double* __restrict__ sc_all,
+                                                               const double* __restrict__ pmax,
+                                                               double* __restrict__ out) {
+    constexpr int CW = 64, CS = HD / CW;  // value columns of a workgroup, workgroups per head
+    constexpr int DB = CW / 32, PP = kChunkP + 2, F4 = kChunkP * CW / 4 / 256;
+    static_assert(HD % CW == 0, "64-column slices");
+    __shared__ __align__(16) double sv[kChunkP * CW];
+    __shared__ __align__(16) double sp[kTileQ * PP];
+    __shared__ double s_es[kTileQ];
+    const int tid = threadIdx.x;
+    const int h = blockIdx.x / CS, col0 = (blockIdx.x % CS) * CW;
+    const int tile = gridDim.y - 1 - blockIdx.y;  // longest tiles first
+    const int b = blockIdx.z;
+    const int s0 = tile * kTileQ;
+    const int nq = min(kTileQ, seq - s0);
+    const int base = *pos0;
+    const int q_dim = heads * HD, kv_dim = kv_heads * HD;
+    const int kvh = h / (heads / kv_heads);
+    const size_t row0 = (size_t)b * seq + s0;
+    if (base + s0 + nq > span) {
+        for (int i = tid; i < nq * CW; i += 256)
+            out[(row0 + i / CW) * q_dim + (size_t)h * HD + col0 + i % CW] = __builtin_nan("");
+        return;
+    }
+    const int nch = (base + s0 + nq + kChunkP - 1) / kChunkP;
+    const float* vb = cache_v + (size_t)b * msl * kv_dim + (size_t)kvh * HD + col0;
+    const int qp = tid >> 4, pp = tid & 15;
+    const int qa = 2 * qp;
+    const int lim_a = base + s0 + qa;
+    const bool w1 = qa + 1 < nq;
+    // (rows past the tile's last query read the last query's scores, unused)
+    const size_t rowa = (row0 + min(qa, nq - 1)) * heads + h;
+    const double* sca = sc_all + rowa * (size_t)span;
+    const size_t sc_next = w1 ? (size_t)heads * span : 0;
+    const double* pma = pmax + rowa * kScoreParts;
+    const double* pmb = pma + (w1 ? (size_t)heads * kScoreParts : 0);
+    double m0 = -1e9, m1 = -1e9;
+#pragma unroll
+    for (int i = 0; i < kScoreParts; ++i) {
+        m0 = pma[i] > m0 ? pma[i] : m0;
+        m1 = pmb[i] > m1 ? pmb[i] : m1;
+    }
+    const int pq = tid >> 5, dl = tid & 31;
+    double acc[4][DB];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < DB; ++j) acc[i][j] = 0.0;
+    double es = 0.0;  // lane tid < kTileQ: query tid
+    float4 rv[F4];
+    auto load = [&](int c) {
+#pragma unroll
+        for (int j = 0; j < F4; ++j) {
+            const int e = (tid + j * 256) * 4;
+            rv[j] = *(const float4*)(vb + (size_t)min(c * kChunkP + e / CW, msl - 1) * kv_dim + e % CW);
+        }
+    };
+    double sv00, sv01, sv10, sv11;
+    auto load_scores = [&](int c) {
+        const int k = min(c, nch - 1) * kChunkP + pp;
+        const int k0c = min(k, span - 1), k1c = min(k + 16, span - 1);
+        sv00 = sca[k0c];
+        sv01 = sca[k1c];
+        sv10 = sca[sc_next + k0c];
+        sv11 = sca[sc_next + k1c];
+    };
+    load(0);
+    load_scores(0);
+    // every query of the tile sees every position of chunks before this one
+    const int whole_ch = (base + s0 + 1) / kChunkP;
+    const double* pe = &sp[min(tid, kTileQ - 1) * PP];  // expSum row (wave 0)
+    const double* vr = &sv[2 * dl];
+    for (int c = 0; c < nch; ++c) {
+#pragma unroll
+        for (int j = 0; j < F4; ++j) {  // V chunk, row-major: v[position][d]
+            const int e = (tid + j * 256) * 4;
+            double* d = &sv[e];
+            *(double2*)d = make_double2((double)rv[j].x, (double)rv[j].y);
+            *(double2*)(d + 2) = make_double2((double)rv[j].z, (double)rv[j].w);
+        }
+        const int k = c * kChunkP + pp;
+        sp[qa * PP + pp] = k <= lim_a ? exp(sv00 - m0) : 0.0;
+        sp[qa * PP + pp + 16] = k + 16 <= lim_a ? exp(sv01 - m0) : 0.0;
+        sp[(qa + 1) * PP + pp] = k <= lim_a + 1 ? exp(sv10 - m1) : 0.0;
+        sp[(qa + 1) * PP + pp + 16] = k + 16 <= lim_a + 1 ? exp(sv11 - m1) : 0.0;
+        load(min(c + 1, nch - 1));  // next V chunk
+        load_scores(c + 1);
+        tile_lds_barrier();  // chunk c's values and probabilities staged
+        const int kc = c * kChunkP;
+        if (c < whole_ch) {  // wave-uniform
+            if (tid < 64)
+                tile_pv_whole<CW, true>(&sp[4 * pq * PP], pe, vr, acc, es);
+            else
+                tile_pv_whole<CW, false>(&sp[4 * pq * PP], pe, vr, acc, es);
+        } else {
+            tile_pv_masked<CW>(&sp[4 * pq * PP], pe, vr, base + s0 + 4 * pq - kc, base + s0 + tid - kc, acc, es);
+        }
+        tile_lds_barrier();  // chunk c's reads done before chunk c + 1 is staged
+    }
+    if (tid < kTileQ) s_es[tid] = es;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int qi = 4 * pq + i;
+        if (qi < nq) {
+            const double e = s_es[qi];
+            double2* o = (double2*)(out + (row0 + qi) * q_dim + (size_t)h * HD + col0 + 2 * dl);
+            *o = make_double2(acc[i][0] / e, acc[i][1] / e);
         }
     }
 }
@@ -2233,7 +2489,7 @@ size_t attention_scratch_bytes(int rows, int heads, int hd, int span, int strict
         if (hd != 64 && hd != 128) return 0;
         if (!strict && fast_qt == 1) return 0;
         if (!strict && fast_qt == 0) rows = rows < kAutoTwoPassRows ? rows : kAutoTwoPassRows;
-        return (size_t)rows * heads * span * 8;
+        return (size_t)rows * heads * (span + (strict ? kScoreParts : 0)) * 8;
     }
     // (room for 32-position chunks; the 64-position kernels use a prefix of each region)
     const size_t rh = (size_t)rows * heads;
@@ -2341,6 +2597,12 @@ hipError_t launch_attention_rope(const int32_t* acc, const float* amax, float sq
     return hipGetLastError();
 }
 
+// Strict prefill tiles (heads x query tiles x sequences) up to which the two
+// launches are shorter (the BitNet-2B block, one launch against two: 80 tiles
+// 143 -> 129 us, 160 188 -> 161, 320 291 -> 252; 640 equal, 1,280 1,668 against
+// 1,734).
+constexpr int kSplitTiles = 512;
+
 hipError_t launch_attention(const double* q, const float* cache_k, const float* cache_v,
                             int batch, int seq, const int* pos0, int msl, int span, int heads,
                             int kv_heads, int hd, int strict, int fast_qt, double* scratch,
@@ -2418,6 +2680,22 @@ hipError_t launch_attention(const double* q, const float* cache_k, const float* 
 #define LAMD_FAST(HDV, QTV)                                                                          \
     hipLaunchKernelGGL((attn_tile_mfma_kernel<HDV, QTV>), gridf, dim3(256), 0, s, q, cache_k, cache_v, \
                        pos0, msl, span, heads, kv_heads, seq, scratch, out)
+        if (strict && (long)grid.x * grid.y * grid.z <= tune_int("LOOM_AMD_ATTN_SPLIT", kSplitTiles)) {
+            double* pm = scratch + (size_t)rows * heads * span;
+            const dim3 ga(heads, grid.y, batch * kScoreParts), gb(heads * (hd / 64), grid.y, batch);
+#define LAMD_SPLIT(HDV)                                                                                         \
+    hipLaunchKernelGGL((attn_tile_scores_kernel<HDV>), ga, dim3(256), 0, s, q, cache_k, pos0, msl, span, heads, \
+                       kv_heads, seq, scratch, pm);                                                             \
+    hipLaunchKernelGGL((attn_tile_values_kernel<HDV>), gb, dim3(256), 0, s, cache_v, pos0, msl, span, heads,    \
+                       kv_heads, seq, scratch, pm, out)
+            if (hd == 128) {
+                LAMD_SPLIT(128);
+            } else {
+                LAMD_SPLIT(64);
+            }
+#undef LAMD_SPLIT
+            return hipGetLastError();
+        }
         if (hd == 128) {
             if (strict) {
                 LAMD_TILE(128);

@@ -983,3 +983,27 @@ def test_strict_decode_chains_at_chunk_edges(orc, torch_dev, tf, hd, prompt):
             assert g[b].tobytes() == r[0].tobytes()
     both.release()
     one.release()
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("batch,seq", [(1, 17), (1, 32), (2, 33), (1, 97), (2, 160)])
+def test_strict_prefill_two_launches_equal_one(orc, torch_dev, tf, tuning, hd, batch, seq):
+    # the strict prefill's score and value launches give the bytes of the
+    # one-launch kernel (LOOM_AMD_ATTN_SPLIT=0): partial tiles, tiles of fewer
+    # chunks than the score ranges, whole and partly seen chunks
+    torch = torch_dev
+    sh = Shape(256, 4, 2, hd, 512, 160)
+    w = Weights(orc, sh, seed=1701, act=ACT_SILU)
+    cfg = w.cfg(tf, "strict")
+    cfg.max_batch = 2
+    gw = w.gpu(tf)
+    x_in = orc.normal_f32(batch * seq * sh.hidden, 1702).reshape(batch, seq, sh.hidden)
+    outs = {}
+    for split in (1 << 20, 0):
+        tuning("LOOM_AMD_ATTN_SPLIT", split)
+        blk = tf.BitNetBlock(cfg, gw)
+        x = to_dev(torch, x_in)
+        _, t = blk.forward(x, taps=True)
+        outs[split] = (x.cpu().numpy().tobytes(), t.attn.cpu().numpy().tobytes())
+        blk.release()
+    assert outs[1 << 20] == outs[0]

@@ -39,9 +39,15 @@ NORM_FAST = 0
 TILE_COLS = 256
 
 
+_torch_module = None
+
+
 def _torch():
-    import torch
-    return torch
+    global _torch_module
+    if _torch_module is None:
+        import torch
+        _torch_module = torch
+    return _torch_module
 
 
 def padded_cols(k: int) -> int:
@@ -49,12 +55,16 @@ def padded_cols(k: int) -> int:
 
 
 def _ptr(t):
-    return None if t is None else C.c_void_p(t.data_ptr())
+    return None if t is None else t.data_ptr()
 
 
-def _stream(device: int):
+def _stream(device: int) -> int:
+    # the raw handle of torch's current stream (current_stream() builds a Stream
+    # object around it: 1.1 us of a one-row call's 8)
     torch = _torch()
-    return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    if not torch.cuda.is_initialized():
+        torch.cuda.init()
+    return torch._C._cuda_getCurrentRawStream(device)
 
 
 def _norm_mode(norm) -> int:
@@ -218,7 +228,7 @@ def dense_forward_packed_ternary(w: TernaryMatrix, x, activation: int = ACT_LINE
     if x.dtype != torch.float32 or x.shape[1] != w.cols:
         raise ValueError(f"x must be float32 [M, {w.cols}]")
     m = x.shape[0]
-    pre = out if out is not None else torch.empty((m, w.rows), dtype=torch.float32, device=x.device)
+    pre = out if out is not None else x.new_empty((m, w.rows))
     post = None
     if activation != ACT_LINEAR:
         post = torch.empty_like(pre)
@@ -271,8 +281,8 @@ def swiglu_forward_packed_ternary(gate: TernaryMatrix, up: TernaryMatrix, down: 
     if x.dtype != torch.float32 or x.shape[1] != hidden:
         raise ValueError(f"x must be float32 [M, {hidden}]")
     m = x.shape[0]
-    h = torch.empty((m, inter), dtype=torch.float32, device=x.device)
-    out = torch.empty((m, hidden), dtype=torch.float32, device=x.device)
+    h = x.new_empty((m, inter))
+    out = x.new_empty((m, hidden))
     t = None
     ct = None
     if taps:

@@ -201,6 +201,7 @@ const char* const kTuneNames[] = {
 constexpr int kTuneCount = (int)(sizeof(kTuneNames) / sizeof(kTuneNames[0]));
 
 struct TuneSnapshot {
+    bool any = false;  // no variable set: every lookup gives its default
     bool set[kTuneCount];
     int value[kTuneCount];
 };
@@ -215,6 +216,7 @@ const TuneSnapshot* read_tuning_locked() {
         const char* v = getenv(kTuneNames[i]);
         t->set[i] = v && *v;
         t->value[i] = t->set[i] ? atoi(v) : 0;
+        t->any |= t->set[i];
     }
     g_tune_all.push_back(std::move(t));
     return g_tune_all.back().get();
@@ -232,6 +234,7 @@ int tune_int(const char* name, int dflt) {
             g_tune.store(t, std::memory_order_release);
         }
     }
+    if (!t->any) return dflt;
     for (int i = 0; i < kTuneCount; ++i) {
         if (strcmp(name, kTuneNames[i]) == 0) return t->set[i] ? t->value[i] : dflt;
     }

@@ -202,8 +202,31 @@ void release(loom_accel_compiled_layer* l) {
     delete l;
 }
 
-// Runs the layer on l->d_in -> l->d_out and waits for it.  The caller holds
-// the device's lock: every layer on a device shares its scratch arena and
+// Copies between a layer's pinned staging and its device buffers.  Up to
+// kCopyKernelBytes a kernel on the layer's stream moves them (the pinned memory
+// is mapped): the copy engine's hand-over to and from the kernels costs several
+// microseconds each way.
+constexpr size_t kCopyKernelBytes = (size_t)1 << 20;
+
+__global__ __launch_bounds__(256) void staging_copy_kernel(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst,
+                                                           size_t words) {
+    const size_t quads = words >> 2, stride = (size_t)gridDim.x * 256;
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < quads; i += stride)
+        ((uint4*)dst)[i] = ((const uint4*)src)[i];
+    const size_t tail = (quads << 2) + threadIdx.x;
+    if (blockIdx.x == 0 && tail < words) dst[tail] = src[tail];
+}
+
+hipError_t staging_copy(void* dst, const void* src, size_t bytes, hipMemcpyKind kind, hipStream_t s) {
+    if (bytes > kCopyKernelBytes || bytes == 0) return hipMemcpyAsync(dst, src, bytes, kind, s);
+    const size_t blocks = (bytes / 16 + 255) / 256;
+    hipLaunchKernelGGL(staging_copy_kernel, dim3((unsigned)(blocks ? blocks : 1)), dim3(256), 0, s, (const uint32_t*)src,
+                       (uint32_t*)dst, bytes / 4);
+    return hipGetLastError();
+}
+
+// Queues the layer on l->d_in -> l->d_out.  The caller holds the device's lock
+// until the stream is idle again: every layer on a device shares its scratch arena and
 // split-K workspace (loom's Go glue has no lock of its own, and goroutines
 // may call infer on two compiled layers at once).
 int run(loom_accel_compiled_layer* l, std::string* why) {
@@ -223,11 +246,6 @@ int run(loom_accel_compiled_layer* l, std::string* why) {
     }
     if (rc != 0) {
         *why = loom_amd_last_error();
-        return -1;
-    }
-    hipError_t e = hipStreamSynchronize(l->stream);
-    if (e != hipSuccess) {
-        *why = std::string("hipStreamSynchronize: ") + hipGetErrorString(e);
         return -1;
     }
     return 0;
@@ -402,7 +420,13 @@ int loom_accel_first_infer(loom_accel_compiled_layer* layer, double* first_infer
     }
     std::string why;
     if (run(layer, &why) != 0) {
+        (void)hipStreamSynchronize(layer->stream);
         set_err(err, err_len, why);
+        return -1;
+    }
+    e = hipStreamSynchronize(layer->stream);
+    if (e != hipSuccess) {
+        set_err(err, err_len, std::string("hipStreamSynchronize: ") + hipGetErrorString(e));
         return -1;
     }
     if (first_infer_ms) *first_infer_ms = ms_since(t0);
@@ -429,21 +453,23 @@ int loom_accel_infer(loom_accel_compiled_layer* layer, const void* in, size_t in
     }
     const auto t0 = Clock::now();
     std::lock_guard<std::mutex> lock(lamd::device_mutex(layer->device));
-    // run() leaves the stream idle, so the previous call's copies are done
+    lamd::DeviceGuard guard(layer->device);
+    // every call leaves the stream idle, so the previous call's copies are done
     memcpy(layer->h_in, in, in_bytes);
-    hipError_t e = hipMemcpyAsync(layer->d_in, layer->h_in, in_bytes, hipMemcpyHostToDevice,
-                                  layer->stream);
+    hipError_t e = staging_copy(layer->d_in, layer->h_in, in_bytes, hipMemcpyHostToDevice, layer->stream);
     if (e != hipSuccess) {
         set_err(err, err_len, std::string("infer upload: ") + hipGetErrorString(e));
         return -1;
     }
     std::string why;
     if (run(layer, &why) != 0) {
+        (void)hipStreamSynchronize(layer->stream);
         set_err(err, err_len, why);
         return -1;
     }
-    e = hipMemcpyAsync(layer->h_out, layer->d_out, out_bytes, hipMemcpyDeviceToHost, layer->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(layer->stream);
+    e = staging_copy(layer->h_out, layer->d_out, out_bytes, hipMemcpyDeviceToHost, layer->stream);
+    const hipError_t es = hipStreamSynchronize(layer->stream);  // (also after a failed launch)
+    if (e == hipSuccess) e = es;
     if (e != hipSuccess) {
         set_err(err, err_len, std::string("infer download: ") + hipGetErrorString(e));
         return -1;

@@ -117,6 +117,10 @@ struct GemmGrid {
 // and the last of the tile's workgroups to arrive (a device-scope counter)
 // adds the other slots to its own -- integer adds, so the result is the same
 // in any order -- and runs the epilogue.
+// K halves (KW = 2, half-width tiles of one matrix): 512 threads, waves 0-3 and
+// 4-7 each as above on one half of every stage's columns (a weight load brings
+// the two words of that half); the halves' sums meet in LDS after the last
+// stage and waves 0-3 run the epilogue.
 // The epilogue stores straight from the accumulators: per instruction the
 // two half-waves write 128 contiguous bytes of two rows.
 // EPI: 0 = plain dense (fp32 out only), 1 + EPI_DENSE / EPI_SWIGLU / EPI_ACC =
@@ -150,14 +154,16 @@ __device__ __forceinline__ void wait_vm_lgkm0() {
 // s_waitcnt lgkmcnt(0) only (vmcnt and expcnt at their maxima)
 __device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xc07f); }
 
-template <int NMAT, int EPI, int MI, int NJ>
-__global__ __launch_bounds__(256, 2) void gemm_lds_kernel(MatArgs p, GemmGrid gg) {
+template <int NMAT, int EPI, int MI, int NJ, int KW>
+__global__ __launch_bounds__(256 * KW, 2) void gemm_lds_kernel(MatArgs p, GemmGrid gg) {
     static_assert(NJ >= 1 && NJ * NMAT <= 2, "32-row weight blocks per wave and matrix");
     constexpr int BM = 32 * MI;
-    constexpr int NA = BM / 16;  // copies per thread per stage
-    constexpr int NSTEP = 8;     // MFMA K steps per 256-column stage
+    constexpr int NA = BM / 16 / KW;  // copies per thread per stage
+    constexpr int NSTEP = 8 / KW;     // MFMA K steps per 256-column stage and wave
     constexpr int NB = NMAT * NJ * 2;  // weight loads per thread per stage
+    constexpr int NWD = 4 / KW;        // words of a weight load
     static_assert(MI == 2 || MI == 4, "64- or 128-token tiles");
+    static_assert(KW == 1 || (KW == 2 && MI == 2 && NMAT == 1 && NJ == 1), "K halves on half-width tiles");
     __shared__ __align__(16) int8_t As0[BM * 256];
     __shared__ __align__(16) int8_t As1[BM * 256];
     __shared__ __align__(16) int8_t As2[MI == 2 ? BM * 256 : 16];  // (128-token tiles: two buffers)
@@ -167,7 +173,7 @@ __global__ __launch_bounds__(256, 2) void gemm_lds_kernel(MatArgs p, GemmGrid gg
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    const int wn = wave;
+    const int wn = wave & 3, kw = wave >> 2;  // weight rows; K half of every stage (KW = 2)
     const int l32 = lane & 31, h = lane >> 5;
     const int M = p.e.m;
     const int ktiles = p.ktiles;
@@ -197,7 +203,7 @@ __global__ __launch_bounds__(256, 2) void gemm_lds_kernel(MatArgs p, GemmGrid gg
     const int last = st1 - 1;
     const int m_wg = mt * BM;
     const int nb0 = (ng * 4 + wn) * NJ;  // wave's first 32-row weight block
-    for (int t = tid; t < BM; t += 256) {
+    for (int t = tid; t < BM; t += 256 * KW) {
         const int tok = min(m_wg + t, M - 1);
         const RowScale rs = row_scale(p.e, p.e.amax[tok], p.e.xsum[tok]);
         s_os0[t] = rs.os0;
@@ -215,22 +221,22 @@ __global__ __launch_bounds__(256, 2) void gemm_lds_kernel(MatArgs p, GemmGrid gg
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         const int nt = min(2 * (nb0 + j) + ((lane >> 4) & 1), p.ntiles - 1);
-        woff[j] = (nt * ktiles * 64 + (lane & 15) + 16 * h) * 16;
+        woff[j] = (nt * ktiles * 64 + (lane & 15) + 16 * h) * 16 + (KW == 2 ? 8 * kw : 0);
     }
-    // copy c of this lane fills physical chunk P = 256c + 64*wave + lane of a
+    // copy c of this lane fills physical chunk P = 256 KW c + 64*wave + lane of a
     // stage buffer: row P/16, physical chunk P%16 = logical chunk
     // (P%16) ^ (row%16) of that token row
     int aoff_g[NA];
 #pragma unroll
     for (int c = 0; c < NA; ++c) {
-        const int P = 256 * c + 64 * wave + lane;
+        const int P = 256 * KW * c + 64 * wave + lane;
         const int r = P >> 4;
         const int lc = (P & 15) ^ (r & 15);
         aoff_g[c] = min(m_wg + r, M - 1) * p.ldq + lc * 16;
     }
-    auto issue = [&](int8_t* buf, int stage, uint32_t (&b)[NMAT][NJ][2][4]) {
+    auto issue = [&](int8_t* buf, int stage, uint32_t (&b)[NMAT][NJ][2][NWD]) {
 #pragma unroll
-        for (int c = 0; c < NA; ++c) g64_copy(ares, buf + c * 4096 + wave * 1024, aoff_g[c], stage * 256);
+        for (int c = 0; c < NA; ++c) g64_copy(ares, buf + c * 4096 * KW + wave * 1024, aoff_g[c], stage * 256);
 #pragma unroll
         for (int mat = 0; mat < NMAT; ++mat)
 #pragma unroll
@@ -238,12 +244,19 @@ __global__ __launch_bounds__(256, 2) void gemm_lds_kernel(MatArgs p, GemmGrid gg
 #pragma unroll
                 for (int u = 0; u < 2; ++u) {
                     const __amdgpu_buffer_rsrc_t r = mat == 0 ? wres0 : wres1;
-                    const uint4 w = __builtin_bit_cast(
-                        uint4, __builtin_amdgcn_raw_buffer_load_b128(r, woff[j] + 512 * u, stage * 1024, 0));
-                    b[mat][j][u][0] = w.x;
-                    b[mat][j][u][1] = w.y;
-                    b[mat][j][u][2] = w.z;
-                    b[mat][j][u][3] = w.w;
+                    if constexpr (KW == 2) {  // the words of this wave's K half
+                        const uint2 w = __builtin_bit_cast(
+                            uint2, __builtin_amdgcn_raw_buffer_load_b64(r, woff[j] + 512 * u, stage * 1024, 0));
+                        b[mat][j][u][0] = w.x;
+                        b[mat][j][u][1] = w.y;
+                    } else {
+                        const uint4 w = __builtin_bit_cast(
+                            uint4, __builtin_amdgcn_raw_buffer_load_b128(r, woff[j] + 512 * u, stage * 1024, 0));
+                        b[mat][j][u][0] = w.x;
+                        b[mat][j][u][1] = w.y;
+                        b[mat][j][u][NWD - 2] = w.z;
+                        b[mat][j][u][NWD - 1] = w.w;
+                    }
                 }
     };
 
@@ -258,11 +271,12 @@ __global__ __launch_bounds__(256, 2) void gemm_lds_kernel(MatArgs p, GemmGrid gg
     // lane's A rows l32 and 32 + l32 (immediate +8192); step with chunk pair
     // (c0, c0 + 1) reads logical chunk c0 + h = c0 ^ h at physical chunk
     // c0 ^ h ^ (l32 & 15)
-    const int abase = l32 * 256 + ((h ^ (l32 & 15)) << 4);
-    auto compute = [&](const int8_t* buf, const uint32_t (&bw)[NMAT][NJ][2][4]) {
+    // (KW = 2: the wave's K half is chunks 8 kw ..)
+    const int abase = l32 * 256 + ((h ^ (l32 & 15) ^ (8 * kw)) << 4);
+    auto compute = [&](const int8_t* buf, const uint32_t (&bw)[NMAT][NJ][2][NWD]) {
 #pragma unroll
         for (int idx = 0; idx < NSTEP; ++idx) {
-            const int hh = idx >> 2, q = idx & 3;
+            const int hh = idx >> 2, q = idx & 3;  // (KW = 2: hh = 0, the wave's own half)
             const int c0 = hh * 8 + (q & 1) * 4 + (q >> 1) * 2;
             const int off = abase ^ (c0 << 4);
             v4i a[MI];
@@ -310,7 +324,7 @@ __global__ __launch_bounds__(256, 2) void gemm_lds_kernel(MatArgs p, GemmGrid gg
     // copies, so a count that relied on the order inside one issue could let
     // copies of the stage about to be read through.)
     constexpr int kAfter = NA + NB;
-    uint32_t bw0[NMAT][NJ][2][4], bw1[NMAT][NJ][2][4], bw2[NMAT][NJ][2][4];
+    uint32_t bw0[NMAT][NJ][2][NWD], bw1[NMAT][NJ][2][NWD], bw2[NMAT][NJ][2][NWD];
     if constexpr (MI == 4) {
         // 128-token tiles: two 32 KB stage buffers (two workgroups per CU),
         // stage s+1 copied while stage s is computed
@@ -367,7 +381,38 @@ __global__ __launch_bounds__(256, 2) void gemm_lds_kernel(MatArgs p, GemmGrid gg
     }
     wait_vm_lgkm0<0>();  // no copy may still be writing LDS when the workgroup ends
 
-    if (MI == 2 && S > 1) {
+    if constexpr (KW == 2) {
+        // the K halves meet: waves 4-7 hand their sums to waves 0-3 through the
+        // stage buffers (block i in buffer i; integer sums, so exact in any
+        // order) and are done
+        __builtin_amdgcn_s_barrier();  // every wave has read its last stage
+        v4i* const x0 = (v4i*)As0 + wn * 256 + lane;
+        v4i* const x1 = (v4i*)As1 + wn * 256 + lane;
+        if (kw == 1) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const v16i &c0 = acc[0][0][0], &c1 = acc[0][1][0];
+                x0[q * 64] = v4i{c0[4 * q], c0[4 * q + 1], c0[4 * q + 2], c0[4 * q + 3]};
+                x1[q * 64] = v4i{c1[4 * q], c1[4 * q + 1], c1[4 * q + 2], c1[4 * q + 3]};
+            }
+        }
+        wait_lgkm0();
+        __asm__ __volatile__("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        __asm__ __volatile__("" ::: "memory");
+        if (kw == 1) return;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const v4i a = x0[q * 64], b = x1[q * 64];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                acc[0][0][0][4 * q + r] += a[r];
+                acc[0][1][0][4 * q + r] += b[r];
+            }
+        }
+    }
+
+    if (KW == 1 && MI == 2 && S > 1) {
         // Slot layout: 16-byte group q (values 4q .. 4q+3) of accumulator
         // block b of thread t at int offset ((b*4 + q)*256 + t)*4, so each
         // store or load instruction of the workgroup covers 4 KB in one run.
@@ -714,6 +759,16 @@ constexpr int kSplitTarget = 240;
 constexpr int kMinSplitKtiles = 6;
 constexpr int kMaxSplit = 4;
 
+// Eight waves a half-width tile, each four on one K half of every stage, where
+// the workgroups do not share their CUs (at most kHalfKMaxTiles) and K is long:
+// with four waves a CU one wave a SIMD waits out every operand read and
+// barrier, about 1,000 cycles a stage of 512 MFMA cycles.  N = 2560, K = 6912:
+// 300 rows 15.7 -> 14.3 us, 512 rows 15.5 -> 14.0 (two more stages of prefetch
+// instead: no change).  At K = 2560 both take the same, at K = 1000 the halves'
+// exchange costs 0.3 us, hence kHalfKMinKtiles.
+constexpr int kHalfKMaxTiles = 256;
+constexpr int kHalfKMinKtiles = 16;
+
 struct GemmPlan {
     int mi, ksplit, sps, nj;
 };
@@ -751,7 +806,7 @@ static GemmPlan plan_gemm(int m, int ntiles, int ktiles, int nmat, int device) {
     return GemmPlan{2, ks, ks > 1 ? sps : ktiles, nj};
 }
 
-template <int NMAT, int EPI, int MI, int NJ>
+template <int NMAT, int EPI, int MI, int NJ, int KW = 1>
 static hipError_t launch_gemm_tile(const MatArgs& p, const GemmPlan& pl, int device, hipStream_t s) {
     GemmGrid gg;
     gg.mtiles = ceil_div(p.e.m, 32 * MI);
@@ -764,7 +819,7 @@ static hipError_t launch_gemm_tile(const MatArgs& p, const GemmPlan& pl, int dev
     gg.ctr = ws.ctr;
     const int total = gg.mtiles * gg.ngroups * gg.ksplit;
     const int grid = ceil_div(total, kXcds) * kXcds;
-    hipLaunchKernelGGL((gemm_lds_kernel<NMAT, EPI, MI, NJ>), dim3(grid), dim3(256), 0, s, p, gg);
+    hipLaunchKernelGGL((gemm_lds_kernel<NMAT, EPI, MI, NJ, KW>), dim3(grid), dim3(256 * KW), 0, s, p, gg);
     return hipGetLastError();
 }
 
@@ -773,6 +828,10 @@ static hipError_t launch_gemm_planned(const MatArgs& p, int device, hipStream_t 
     const GemmPlan pl = plan_gemm(p.e.m, p.ntiles, p.ktiles, NMAT, device);
     if (pl.mi == 4) return launch_gemm_tile<NMAT, EPI, 4, 2 / NMAT>(p, pl, device, s);
     if constexpr (NMAT == 1) {
+        const int tiles = ceil_div(p.e.m, 64) * ceil_div(p.ntiles, 8);
+        if (pl.nj == 1 && pl.ksplit == 1 && p.ktiles >= kHalfKMinKtiles &&
+            tiles <= tune_int("LOOM_AMD_GEMM_KHALF", kHalfKMaxTiles))
+            return launch_gemm_tile<1, EPI, 2, 1, 2>(p, pl, device, s);
         if (pl.nj == 1) return launch_gemm_tile<1, EPI, 2, 1>(p, pl, device, s);
     }
     return launch_gemm_tile<NMAT, EPI, 2, 2 / NMAT>(p, pl, device, s);

@@ -866,6 +866,20 @@ def test_gemm_half_width_tiles(orc, torch_dev, bn, tuning, nj, split, rows, cols
     _check_dense(orc, torch_dev, bn, m, x, activation=0, residual=res)
 
 
+@pytest.mark.parametrize("rows,cols,M", [(130, 4000, 65), (512, 4300, 129), (1000, 4608, 300), (2560, 6912, 512)])
+def test_gemm_k_halves(orc, torch_dev, bn, tuning, rows, cols, M):
+    # half-width tiles whose eight waves halve every K stage (16 or more K
+    # tiles): 16, 17, 18 and 27 stages (each tail of the three-stage loop),
+    # ragged columns, weight rows and token rows, plain and with residual + ReLU
+    tuning("LOOM_AMD_GEMM_NJ", "1")
+    tuning("LOOM_AMD_GEMM_SPLIT", "1")
+    m = orc.random_matrix(rows, cols, seed=rows + cols + M)
+    x = orc.normal_f32(M * cols, seed=M + 21).reshape(M, cols)
+    res = orc.normal_f32(M * rows, seed=M + 22).reshape(M, rows)
+    _check_dense(orc, torch_dev, bn, m, x)
+    _check_dense(orc, torch_dev, bn, m, x, activation=0, residual=res)
+
+
 @pytest.mark.parametrize("n", [2560, 6912, 1000, 260, 8192, 4, 1001])
 def test_norm_quant_rows_one_wave_equal_workgroup(orc, torch_dev, bn, tuning, n):
     # fast inner norm + requantization of 1024 or more rows, one wave per row,

@@ -3006,17 +3006,20 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const float* __restrict__ 
 //    output, in one lane;
 //  - sequential: k = g takes column 4 m + g (one dword a lane).
 // A wave owns 16 vocab rows (B) and 16 MT rows of x (A), 256 threads four
-// such waves; x goes through LDS in slabs of 128 columns (pitch 132: the 16
-// rows that a 16-byte read covers fall in distinct banks), the table straight
-// to registers, four steps ahead of their MFMAs (2 KB a wave and step: 96 KB
-// in flight a CU at three waves per SIMD).  The barriers wait for LDS only, so
-// the table loads stay in flight across them.
+// such waves; x goes through LDS in slabs of 128 columns, as doubles: each
+// value is converted once a workgroup and not by every wave that reads it
+// (held as floats 2-16 rows took 302-315 us, 17-32 rows 403-409, sequential
+// 655-673).  Pitch 130: the 16 rows that a 16-byte read covers fall in
+// distinct banks.  The table goes straight to registers, four steps ahead of
+// its MFMAs (2 KB a wave and step: 96 KB in flight a CU at three waves per
+// SIMD).  The barriers wait for LDS only, so the table loads stay in flight
+// across them.
 // Bound: HBM for one 16-row tile (1.31 GB at vocab 128256 x 2560: 195 us at
 // the 6.7 TB/s of the one-row kernel; 145 us of MFMA issue): 2 to 16 rows take
-// 302-315 us, against 195 us a row (16 rows 3,066 us) with the one-row kernel
+// 298-312 us, against 195 us a row (16 rows 3,066 us) with the one-row kernel
 // reading the table once per row.  MT = 2 from 17 rows (the table read once
-// for 32 rows, 409 us; two MT = 1 tiles would take twice 302).  Sequential order:
-// 655-673 us (its one chain per output waits on every MFMA).
+// for 32 rows, 391 us; two MT = 1 tiles would take twice 298).  Sequential order:
+// 613-651 us (its one chain per output waits on every MFMA).
 // Padding columns are zero in both operands (0 * Inf never arises; a chain
 // starts at +0 and so never holds -0, which + 0 would change); rows past
 // `rows` and vocab rows past the table are computed and not stored.
@@ -3024,7 +3027,7 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const float* __restrict__ 
 
 typedef double v4d_head __attribute__((ext_vector_type(4)));
 constexpr int kHeadCols = 128;            // columns per x slab: four steps of 32
-constexpr int kHeadPitch = kHeadCols + 4;
+constexpr int kHeadPitch = kHeadCols + 2;
 constexpr int kHeadAhead = 4;             // table steps in flight
 
 template <bool VEC, bool DOTTILE, int MT>
@@ -3032,7 +3035,7 @@ __global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restri
                                                            const float* __restrict__ x, int rows,
                                                            float* __restrict__ logits) {
     static_assert(kHeadCols == 32 * kHeadAhead, "a slab is one turn of the table ring");
-    __shared__ __align__(16) float xs[2][16 * MT * kHeadPitch];
+    __shared__ __align__(16) double xs[2][16 * MT * kHeadPitch];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int r = lane & 15, g = lane >> 4;
     const int v0 = (blockIdx.x * 4 + wave) * 16;
@@ -3070,10 +3073,13 @@ __global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restri
             }
         }
     };
-    auto store_x = [&](float* buf) {
+    auto store_x = [&](double* buf) {
 #pragma unroll
-        for (int i = 0; i < NX; ++i)
-            *(uint4*)&buf[(xr0 + 8 * i) * kHeadPitch + xc] = make_uint4(xn[i][0], xn[i][1], xn[i][2], xn[i][3]);
+        for (int i = 0; i < NX; ++i) {
+            double* d = &buf[(xr0 + 8 * i) * kHeadPitch + xc];
+            *(double2*)d = make_double2((double)__uint_as_float(xn[i][0]), (double)__uint_as_float(xn[i][1]));
+            *(double2*)(d + 2) = make_double2((double)__uint_as_float(xn[i][2]), (double)__uint_as_float(xn[i][3]));
+        }
     };
     // the eight table values of this lane for the step at column c0: chunk g
     // (DotTile), or columns 4 m + g (sequential); columns past ncols read 0
@@ -3101,14 +3107,17 @@ __global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restri
     for (int l = 0; l < NC; ++l)
 #pragma unroll
         for (int t = 0; t < MT; ++t) acc[l][t] = v4d_head{0.0, 0.0, 0.0, 0.0};
-    auto step = [&](const float* buf, int cs, const uint32_t (&w)[8]) {
+    auto step = [&](const double* buf, int cs, const uint32_t (&w)[8]) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
-            const float* xb = buf + (16 * t + r) * kHeadPitch + cs;
-            float a[8];
+            const double* xb = buf + (16 * t + r) * kHeadPitch + cs;
+            double a[8];
             if (DOTTILE) {
-                const float4 p = *(const float4*)(xb + 8 * g), q = *(const float4*)(xb + 8 * g + 4);
-                a[0] = p.x, a[1] = p.y, a[2] = p.z, a[3] = p.w, a[4] = q.x, a[5] = q.y, a[6] = q.z, a[7] = q.w;
+#pragma unroll
+                for (int l = 0; l < 8; l += 2) {
+                    const double2 p = *(const double2*)(xb + 8 * g + l);
+                    a[l] = p.x, a[l + 1] = p.y;
+                }
             } else {
 #pragma unroll
                 for (int l = 0; l < 8; ++l) a[l] = xb[4 * l + g];
@@ -3116,7 +3125,7 @@ __global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restri
 #pragma unroll
             for (int l = 0; l < 8; ++l)
                 acc[DOTTILE ? l : 0][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(
-                    (double)a[l], (double)__uint_as_float(w[l]), acc[DOTTILE ? l : 0][t], 0, 0, 0);
+                    a[l], (double)__uint_as_float(w[l]), acc[DOTTILE ? l : 0][t], 0, 0, 0);
         }
     };
 
@@ -3130,7 +3139,7 @@ __global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restri
     tile_lds_barrier();
     for (int i = 0; i < nslab; ++i) {
         const int c0 = i * kHeadCols;
-        const float* buf = xs[i & 1];
+        const double* buf = xs[i & 1];
         load_x(c0 + kHeadCols);  // (all zero past the last column)
         // the last slab loads its own columns again rather than branch
         const int cn = i + 1 < nslab ? c0 + kHeadCols : c0;

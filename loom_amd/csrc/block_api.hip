@@ -791,14 +791,14 @@ void loom_amd_model_release(loom_amd_model* m) {
 // int8 codes once a row) or forms every logit in one pass over the fp32 table.
 // Measured in us on gfx950 (hidden 2560; x = entries over those of vocab
 // 128256): a screened row 28 + 50 x (three short launches and the codes), the
-// full head of 2 to 16 rows and its pick 20 + 302 x (655 x in sequential
+// full head of 2 to 16 rows and its pick 20 + 298 x (630 x in sequential
 // order), of one row 20 + 195 x and more than the screened row for every table
 // that a model has.
 static bool head_screens(const loom_amd_model* m, int batch) {
     if (!m->lm_q || tune_int("LOOM_AMD_LM_SCREEN", 1) == 0) return false;
     if (batch == 1) return true;
     const double x = (double)m->vocab * m->hidden / (128256.0 * 2560.0);
-    return batch * (28.0 + 50.0 * x) <= 20.0 + (m->lm_sequential ? 655.0 : 302.0) * x * ceil_div(batch, 16);
+    return batch * (28.0 + 50.0 * x) <= 20.0 + (m->lm_sequential ? 630.0 : 298.0) * x * ceil_div(batch, 16);
 }
 
 // Final norm + LM head + argmax of each sequence's last row (row stride ld

@@ -543,7 +543,7 @@ __device__ __forceinline__ double ordered_sum_core(Get get, int n, double s0, Or
         int e = (int)((unsigned long long)__double_as_longlong(lo) >> 52);  // biased exponent
         const bool sq = !(lo >= 0x1p-960 && hi < 0x1p1000 &&
                           e == (int)((unsigned long long)__double_as_longlong(hi) >> 52));
-        const bool negative = __builtin_amdgcn_ballot_w64(!(mn >= 0.0)) != 0ull;
+        const bool negative = !(s0 >= 0.0) || __builtin_amdgcn_ballot_w64(!(mn >= 0.0)) != 0ull;
         if (sq) e = 1023;
         const double scale = __longlong_as_double((long long)(2098 - e) << 52);  // 1/q
         const double q = __longlong_as_double((long long)(e - 52) << 52);
@@ -673,9 +673,11 @@ __device__ __forceinline__ double ordered_sum_core(Get get, int n, double s0, Or
 // integers below 2^52), where each lane's parity comes from wave ballots, and
 // whose sum for an odd incoming parity differs only at its first tie.  Wave 0
 // then walks the records in order: a segment adds its sum (the running sum's
-// parity picks the variant), a sequential lane its terms.  A row with a
-// negative term (the estimate bounds non-negative ones only), or with more
-// records than the slots, goes through ordered_sum_wave.
+// parity picks the variant), a sequential lane its terms.  The walk has no
+// check of its own, so what the estimate does not bound goes through
+// ordered_sum_wave: a row with a negative term or a start that is negative or
+// NaN (large values that cancel leave the estimate an error of any size beside
+// the small sums that follow), and one with more records than the slots.
 //
 // What bounds it is latency.  Stamps of the cycle counter on gfx950 (6,912
 // squares of normal values, eight waves, 24 records): the terms and their plain

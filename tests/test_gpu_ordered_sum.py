@@ -138,6 +138,26 @@ def test_ordered_sum_rows_bit_exact(torch_dev, kind, threads):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("threads", [64, 256, 512])
+@pytest.mark.parametrize("n", [1000, 2560, 6912, 8064])
+def test_ordered_sum_rows_negative_start(torch_dev, n, threads):
+    # a negative start that the first term cancels: an estimate of the running
+    # sums keeps the roundings of the large values, so it is off by up to 2^-25
+    # of the small ones that follow, which pass a power of two within that
+    # distance of a multiple of 1, 3, 5, ... terms (where a lane's block begins)
+    rng = np.random.default_rng(n)
+    rows = 400
+    t = rng.random((rows, n))
+    for r in range(rows):
+        cut = int(rng.integers(1, n // 165)) * 165  # 165 = 3 * 5 * 11
+        t[r] *= (2.0 ** -33) * (1.0 + rng.uniform(-1, 1) * 2.0 ** -27) / t[r, 1:cut].sum()
+    t[:, 0] = 2.0
+    for s0 in (-2.0, np.nan, -np.inf):
+        got, want = gpu_ordered_sums(torch_dev, t, s0, threads), sequential(t, s0)
+        assert same_bits(got, want), (s0, np.nonzero(got.view(np.uint64) != want.view(np.uint64))[0][:8])
+
+
+@pytest.mark.gpu
 def test_ordered_sum_rows_many_rows(torch_dev):
     # BitNet-2B widths, 512 rows each (the strict norms' inputs: fp32 squares)
     rng = np.random.default_rng(3)

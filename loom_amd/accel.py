@@ -116,9 +116,9 @@ class CompiledLayer:
         if inv.nbytes != self._in or outv.nbytes != self._out:
             raise AccelError(f"accel: buffer size mismatch in={inv.nbytes} want={self._in} "
                              f"out={outv.nbytes} want={self._out}")
-        # (a writable buffer is passed as it is, a read-only one is copied)
-        in_type = C.c_char * inv.nbytes
-        in_buf = in_type.from_buffer_copy(inv) if inv.readonly else in_type.from_buffer(inv)
+        # copied while the GIL is held: the call may wait for another layer's,
+        # and the caller may refill its array meanwhile
+        in_buf = (C.c_char * inv.nbytes).from_buffer_copy(inv)
         out_buf = (C.c_char * outv.nbytes).from_buffer(outv) if not outv.readonly else None
         if out_buf is None:
             raise AccelError("accel: output buffer is read-only")

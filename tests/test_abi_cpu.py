@@ -107,6 +107,28 @@ def test_python_accel_mirror_refuses_cpu(amd_lib):
     assert accel.npu_available() == gpu_visible()
 
 
+def test_infer_copies_its_input_when_called():
+    # the rows of the call are those the array held when it was made, also when
+    # the call waits and another thread refills the array (played by an API that
+    # refills it before it reads)
+    import numpy as np
+    from loom_amd import accel
+
+    x, out, seen = np.arange(4, dtype=np.float32), np.zeros(4, np.float32), []
+
+    class Api:
+        def loom_accel_infer(self, handle, inp, in_bytes, outp, out_bytes, ms, err, err_len):
+            x[:] = -1.0
+            seen.append(C.string_at(inp, in_bytes))
+            C.memmove(outp, inp, out_bytes)
+            return 0
+
+    layer = accel.CompiledLayer(Api(), 1, x.nbytes, out.nbytes)
+    layer.infer(x, out)
+    assert np.frombuffer(seen[0], np.float32).tolist() == [0.0, 1.0, 2.0, 3.0]
+    assert out.tolist() == [0.0, 1.0, 2.0, 3.0]
+
+
 def test_c_loader_conformance(amd_lib, tmp_path):
     from loom_amd import _lib
     exe = tmp_path / "abi_conformance"

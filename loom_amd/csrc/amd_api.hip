@@ -197,7 +197,8 @@ const char* const kTuneNames[] = {
     "LOOM_AMD_SKINNY_NT",   "LOOM_AMD_SKINNY_NTR",   "LOOM_AMD_FUSED_NTR",    "LOOM_AMD_FUSED_WAVES",
     "LOOM_AMD_GEMV_STREAM", "LOOM_AMD_STREAM_WAVES", "LOOM_AMD_STREAM_DEPTH", "LOOM_AMD_ATTN_QT",
     "LOOM_AMD_UNFUSED_ROPE", "LOOM_AMD_UNFUSED_NORM", "LOOM_AMD_GEMM_NJ", "LOOM_AMD_ROWNORM_WAVE",
-    "LOOM_AMD_QUANT_GROUPS", "LOOM_AMD_LM_SCREEN", "LOOM_AMD_ROWNORM_BLOCK", "LOOM_AMD_ATTN_SPLIT", "LOOM_AMD_GEMM_KHALF"};
+    "LOOM_AMD_QUANT_GROUPS", "LOOM_AMD_LM_SCREEN", "LOOM_AMD_ROWNORM_BLOCK", "LOOM_AMD_ATTN_SPLIT", "LOOM_AMD_GEMM_KHALF",
+    "LOOM_AMD_FUSED_PAIR"};
 constexpr int kTuneCount = (int)(sizeof(kTuneNames) / sizeof(kTuneNames[0]));
 
 struct TuneSnapshot {
@@ -597,7 +598,7 @@ int loom_amd_swiglu_forward(const loom_amd_matrix* gate, const loom_amd_matrix* 
     gu.ldo = inter;
     gu.acc0 = taps ? taps->acc_gate : nullptr;
     gu.acc1 = taps ? taps->acc_up : nullptr;
-    const bool fused = fused_quant_ok(m, hidden, x, true);
+    const bool fused = fused_quant_ok(m, hidden, x, G.ntiles);
     hipError_t e;
     if (fused) {
         e = launch_matmul_fused(&G, &U, x, m, gu, taps ? taps->xq : nullptr,

@@ -96,9 +96,11 @@ hipError_t launch_act_quant_f64(const double* x, int ldx, int m, int k, int8_t* 
 hipError_t launch_matmul(const Matrix* w0, const Matrix* w1, const QuantAct& a, int m,
                          const Epilogue& epi, hipStream_t s);
 // Same, quantizing fp32 rows x (M x K, row stride K) inside the matmul kernel
-// (one launch).  Only for the shapes fused_quant_ok accepts.  xq_tap (M x K)
-// and amax_tap (M) optionally receive the quantized rows.
-bool fused_quant_ok(int m, int k, const float* x, bool two = false);
+// (one launch).  Only for the shapes fused_quant_ok accepts; for a pair,
+// pair_tiles (the weight tiles of each matrix) also asks whether one launch is
+// the shorter form.  xq_tap (M x K) and amax_tap (M) optionally receive the
+// quantized rows.
+bool fused_quant_ok(int m, int k, const float* x, int pair_tiles = 0);
 hipError_t launch_matmul_fused(const Matrix* w0, const Matrix* w1, const float* x, int m,
                                const Epilogue& epi, int8_t* xq_tap, float* amax_tap,
                                hipStream_t s);

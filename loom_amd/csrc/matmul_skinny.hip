@@ -1240,14 +1240,14 @@ static void launch_fused_w(const MatArgs& p, size_t shm, hipStream_t s) {
 // half the CUs, as for one row (BitNet-2B up shape, M = 8: 6.0 us per Dense
 // step; one tile 7.5, four 7.5; the separate quantization launch took 8.0).
 // LOOM_AMD_FUSED_NTR = 1 or 2 overrides.
-template <int FV>
+template <int NMAT, int FV>
 static void launch_fused_rows_fv(const MatArgs& p, size_t shm, hipStream_t s) {
-    const int ntr = tune_int("LOOM_AMD_FUSED_NTR", ceil_div(p.ntiles, 2) >= 128 ? 2 : 1);
-    if (ntr == 2) {
-        hipLaunchKernelGGL((skinny_kernel<1, 1, 8, true, NORM_NONE, 0, FV, kFusedWaveRows, 2>),
+    const int ntr = NMAT == 1 ? tune_int("LOOM_AMD_FUSED_NTR", ceil_div(p.ntiles, 2) >= 128 ? 2 : 1) : 1;
+    if (NMAT == 1 && ntr == 2) {
+        hipLaunchKernelGGL((skinny_kernel<NMAT, 1, 8, true, NORM_NONE, 0, FV, kFusedWaveRows, 2>),
                            dim3(ceil_div(p.ntiles, 2)), dim3(512), shm, s, p);
     } else {
-        hipLaunchKernelGGL((skinny_kernel<1, 1, 8, true, NORM_NONE, 0, FV, kFusedWaveRows, 1>),
+        hipLaunchKernelGGL((skinny_kernel<NMAT, 1, 8, true, NORM_NONE, 0, FV, kFusedWaveRows, 1>),
                            dim3(p.ntiles), dim3(512), shm, s, p);
     }
 }
@@ -1258,16 +1258,13 @@ static hipError_t launch_skinny(const MatArgs& p, hipStream_t s) {
     constexpr int kCap = NMAT == 1 ? 16 : 8;
     if constexpr (FUSEQ) {
         if (p.e.m > kFusedMaxRows) {  // one row per wave (fused_quant_ok: K <= 4096)
-            if constexpr (NMAT == 1) {
-                const size_t shm = (size_t)p.e.m * p.ldq;
-                if (p.k / 4 <= 10 * 64) {
-                    launch_fused_rows_fv<10>(p, shm, s);
-                } else {
-                    launch_fused_rows_fv<16>(p, shm, s);
-                }
-                return hipGetLastError();
+            const size_t shm = (size_t)p.e.m * p.ldq;
+            if (p.k / 4 <= 10 * 64) {
+                launch_fused_rows_fv<NMAT, 10>(p, shm, s);
+            } else {
+                launch_fused_rows_fv<NMAT, 16>(p, shm, s);
             }
-            return hipErrorInvalidValue;  // (a pair quantizes five or more rows apart)
+            return hipGetLastError();
         }
     }
     int w = pick_waves(p.ntiles, p.ktiles, kCap);
@@ -1465,13 +1462,20 @@ hipError_t launch_matmul(const Matrix* w0, const Matrix* w1, const QuantAct& a, 
     return launch_gemm(p, two, w0->device, s);
 }
 
+// Weight tiles up to which a gate|up pair of five to eight rows quantizes them
+// inside its launch.  Every tile's workgroup repeats the quantization, one
+// workgroup a CU: up to 256 tiles that is one round and saves the launch, above
+// it the second round costs more.  FFN call in us, apart -> fused, five to
+// eight rows, back to back: inter 1,024 to 4,096 at hidden 512 to 2,560 19.0 ->
+// 15.5, 3,072 19.1 -> 16.9, 4,096 19.2 -> 17.4-18.7; inter 5,504 at hidden 512
+// 18.9 -> 18.9-19.6, 1,536 19.1 -> 20.3, 4,096 21.5 -> 25-27; inter 6,912 at
+// hidden 2,560 19.6-20.6 -> 21.5-22.3.
+constexpr int kFusedPairTiles = 256;
+
 // The fused prologue holds the M x K rows in registers (kFusedVec float4 per
 // thread of a 512-thread workgroup) and their int8 copy in LDS.
-// Five to eight rows only for one matrix: a pair quantizes them apart (8 rows
-// at the BitNet-2B gate|up shape: 14.9 us fused; quantization 2.5 us and the
-// plain pair 7.7 us).
-bool fused_quant_ok(int m, int k, const float* x, bool two) {
-    if (two && m > kFusedMaxRows) return false;
+bool fused_quant_ok(int m, int k, const float* x, int pair_tiles) {
+    if (m > kFusedMaxRows && pair_tiles > 0 && pair_tiles > tune_int("LOOM_AMD_FUSED_PAIR", kFusedPairTiles)) return false;
     if (m < 1 || k % 4 != 0 || ((uintptr_t)x & 15) != 0) return false;
     if (m <= kFusedMaxRows)
         return (size_t)m * k <= (size_t)4 * kFusedVec * 512 && pad_cols(k) * (size_t)m <= 64 * 1024;
@@ -1576,7 +1580,7 @@ hipError_t launch_matmul_fused(const Matrix* w0, const Matrix* w1, const float* 
                                const Epilogue& epi, int8_t* xq_tap, float* amax_tap,
                                hipStream_t s) {
     if (m <= 0) return hipSuccess;
-    if (!fused_quant_ok(m, w0->cols, x, epi.kind == EPI_SWIGLU)) return hipErrorInvalidValue;
+    if (!fused_quant_ok(m, w0->cols, x)) return hipErrorInvalidValue;
     MatArgs p = make_args(w0, w1, m, epi);
     p.x = x;
     p.ldq = pad_cols(w0->cols);

@@ -505,6 +505,22 @@ def test_swiglu_row_norm_in_down(orc, torch_dev, bn, norm, shape, tuning):
         assert got[None].tobytes() == got["1"].tobytes()
 
 
+@pytest.mark.parametrize("norm", ["strict", "fast"])
+@pytest.mark.parametrize("hidden,inter,M", [(1024, 2816, 5), (1024, 2816, 8), (260, 4096, 7), (260, 4097, 6), (2564, 4096, 8),
+                                            (4096, 515, 5), (4100, 515, 6)])
+def test_swiglu_pair_of_few_rows(orc, torch_dev, bn, tuning, hidden, inter, M, norm):
+    # five to eight rows: quantized inside the gate and up launch up to 256
+    # weight tiles and 4,096 columns (both widths of the lanes' slots), apart
+    # above either; the same bytes as apart at every size
+    runs = {}
+    for pair in (None, "0"):
+        tuning("LOOM_AMD_FUSED_PAIR", pair)
+        hg, ref = _swiglu_case(orc, torch_dev, bn, hidden=hidden, inter=inter, M=M, seed=1500 + M, norm=norm,
+                               with_norm_w=True)
+        runs[pair] = hg.tobytes()
+    assert runs[None] == runs["0"]
+
+
 @pytest.mark.parametrize("M", [1, 8, 64, 256])
 def test_swiglu_bitnet_2b_shape(orc, torch_dev, bn, M):
     hg, ref = _swiglu_case(orc, torch_dev, bn, hidden=2560, inter=6912, M=M, seed=1234 + M,

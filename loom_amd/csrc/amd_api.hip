@@ -198,7 +198,7 @@ const char* const kTuneNames[] = {
     "LOOM_AMD_GEMV_STREAM", "LOOM_AMD_STREAM_WAVES", "LOOM_AMD_STREAM_DEPTH", "LOOM_AMD_ATTN_QT",
     "LOOM_AMD_UNFUSED_ROPE", "LOOM_AMD_UNFUSED_NORM", "LOOM_AMD_GEMM_NJ", "LOOM_AMD_ROWNORM_WAVE",
     "LOOM_AMD_QUANT_GROUPS", "LOOM_AMD_LM_SCREEN", "LOOM_AMD_ROWNORM_BLOCK", "LOOM_AMD_ATTN_SPLIT", "LOOM_AMD_GEMM_KHALF",
-    "LOOM_AMD_FUSED_PAIR"};
+    "LOOM_AMD_FUSED_PAIR",  "LOOM_AMD_LM_ROWS"};
 constexpr int kTuneCount = (int)(sizeof(kTuneNames) / sizeof(kTuneNames[0]));
 
 struct TuneSnapshot {

@@ -2917,6 +2917,8 @@ __global__ __launch_bounds__(256) void lm_head_kernel(const float* __restrict__ 
     extern __shared__ float xs[];  // hidden
     const int tid = threadIdx.x;
     const int v0 = blockIdx.x * kHeadLogits;
+    x += (size_t)blockIdx.y * hidden;
+    logits += (size_t)blockIdx.y * vocab;
     for (int i = tid; i < hidden; i += 256) xs[i] = x[i];
     constexpr int C4N = kHeadSlab / 4;           // threads per row segment
     constexpr int NL = kHeadLogits * C4N / 256;  // float4 loads per thread per slab
@@ -3085,11 +3087,14 @@ __global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restri
     // (DotTile), or columns 4 m + g (sequential); columns past ncols read 0
     const int wv = (r * hidden + (DOTTILE ? 8 * g : g)) * 4;
     auto load_w = [&](int c0, uint32_t (&w)[8], auto guard) {
-        if constexpr (DOTTILE && VEC && !decltype(guard)::value) {
+        if constexpr (DOTTILE && VEC) {
+            // (ncols is whole chunks: a lane's chunk lies within it or past it)
+            constexpr bool kGuard = decltype(guard)::value;
+            const int off = !kGuard ? wv : c0 + 8 * g < ncols ? wv + 4 * c0 : (int)kPast;
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 const uint4 a = __builtin_bit_cast(
-                    uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, wv + 16 * q, c0 * 4, kLoadNT));
+                    uint4, __builtin_amdgcn_raw_buffer_load_b128(wres, off + 16 * q, kGuard ? 0 : c0 * 4, kLoadNT));
                 w[4 * q] = a.x, w[4 * q + 1] = a.y, w[4 * q + 2] = a.z, w[4 * q + 3] = a.w;
             }
         } else {
@@ -3176,6 +3181,44 @@ __global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restri
         }
 }
 
+// 16-row tiles of x a workgroup of lm_head_rows_kernel keeps (1 or 2), or 0 where
+// the one-row kernel once per row is shorter (`vec`: it reads the table in 16
+// bytes; us, by rows -> together, vocab as stated).
+// Two tiles when one a workgroup would not be a single round of the chip: at
+// hidden 2560, 17 rows, with one tile and with two: vocab 8,000 39 and 56,
+// 16,000 72 and 57, 128,256 595 and 382; at hidden 300, 40 rows, vocab 4,000 9
+// and 14, 8,000 15 and 14.
+// DotTile order: two rows are shorter together (2,000 at hidden 2560 72 -> 38,
+// 128,256 384 -> 284) but for narrow rows of a large table (hidden 128, 64,000:
+// 10.4 -> 13.2; 300, 128,256: 63 -> 70; but 256, 64,000: 21 -> 19).
+// Sequential order: the single chain of a logit waits on every MFMA, 76 us a
+// round of 256 workgroups at hidden 2560 (the dwords of 16 rows a multiple of 64
+// floats apart cost a fourth more than at other strides: 1340 280 -> 261 where
+// 1280 takes 198 -> 331), so at those strides, and for narrow rows,
+//  - two rows stay apart from the second round on (hidden 2560, 32,000 101 ->
+//    151, 128,256 384 -> 632; 1024 191 -> 261; 300 64 -> 70), three of a large
+//    table too (2560 575 -> 634, 448 102 -> 129) unless a multiple of 1,024
+//    floats apart (1024 279 -> 261, 2048 570 -> 492), up to four of narrow rows
+//    (hidden 128, 32,000: 11.5 -> 15.7),
+//  - and short rows of a small table while each workgroup has a CU (hidden 1024,
+//    4,000 30 -> 34; 576, 8,000 20 -> 22; 2560, three rows 83 -> 75).
+static int head_rows_tile(int vocab, int hidden, int rows, bool dottile, bool vec) {
+    constexpr int kCus = 256;
+    if (rows < 2) return 0;
+    int tiles = rows <= 16 || ceil_div(vocab, 64) * ceil_div(rows, 16) <= kCus ? 1 : 2;
+    const bool narrow = hidden <= 320, large = vocab >= 48000;
+    if (vec && dottile) {
+        if (rows == 2 && narrow && large && hidden % 256 != 0) tiles = 0;
+    } else if (vec && (hidden % 64 == 0 || narrow)) {
+        if (rows == 2 && ceil_div(vocab, 64) > kCus + kCus / 8) tiles = 0;
+        if (rows == 3 && large && hidden % 64 == 0 && hidden % 1024 != 0) tiles = 0;
+        if (rows <= 4 && hidden >= 128 && hidden <= 256) tiles = 0;
+        if (hidden <= 1024 && vocab <= (hidden <= 640 ? 8192 : 6000) && rows * ceil_div(vocab, kHeadLogits) <= kCus)
+            tiles = 0;
+    }
+    return min(max(tune_int("LOOM_AMD_LM_ROWS", tiles), 0), 2);
+}
+
 template <bool DOTTILE>
 static hipError_t launch_head(const float* table, int vocab, int hidden, const float* x, int rows,
                               float* logits, hipStream_t s) {
@@ -3183,9 +3226,9 @@ static hipError_t launch_head(const float* table, int vocab, int hidden, const f
     const size_t shm = (size_t)hidden * sizeof(float);
     if (shm > 64 * 1024) return hipErrorInvalidValue;
     const dim3 b(256);
-    if (rows > 1) {
-        const bool vec = hidden % 8 == 0 && (((uintptr_t)table | (uintptr_t)x) & 15) == 0;
-        const int mt = rows > 16 ? 2 : 1;
+    const bool vect = hidden % 4 == 0 && ((uintptr_t)table & 15) == 0;
+    if (const int mt = head_rows_tile(vocab, hidden, rows, DOTTILE, vect)) {
+        const bool vec = vect && ((uintptr_t)x & 15) == 0;
         const dim3 g((unsigned)ceil_div(vocab, 64), (unsigned)ceil_div(rows, 16 * mt));
 #define LAMD_HEAD_ROWS(V, MTV)                                                                            \
     hipLaunchKernelGGL((lm_head_rows_kernel<V, DOTTILE, MTV>), g, b, 0, s, table, vocab, hidden, x, rows, \
@@ -3200,7 +3243,7 @@ static hipError_t launch_head(const float* table, int vocab, int hidden, const f
 #undef LAMD_HEAD_ROWS
         return hipGetLastError();
     }
-    const dim3 g((unsigned)ceil_div(vocab, kHeadLogits));
+    const dim3 g((unsigned)ceil_div(vocab, kHeadLogits), rows);
     if (hidden % 4 == 0 && ((uintptr_t)table & 15) == 0) {
         hipLaunchKernelGGL((lm_head_kernel<true, DOTTILE>), g, b, shm, s, table, vocab, hidden, x,
                            logits);

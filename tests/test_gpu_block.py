@@ -935,6 +935,33 @@ def test_lm_head_rows_equal_single_rows(torch_dev, tf, sequential, rows, vocab, 
         assert torch.equal(got[r].nan_to_num(0.5), one.nan_to_num(0.5)), r
 
 
+@pytest.mark.parametrize("sequential", [False, True])
+@pytest.mark.parametrize("rows,vocab,hidden", [(2, 65, 12), (3, 130, 132), (2, 64, 140), (17, 63, 300), (33, 200, 260),
+                                               (2, 1000, 1340), (16, 257, 576), (2, 18500, 64)])
+def test_lm_head_forms_agree(torch_dev, tf, tuning, sequential, rows, vocab, hidden):
+    # the form that the rule takes, the one-row kernel once per row and one or two
+    # row tiles a workgroup: the same bits, also where the rows are read in 16
+    # bytes but hold no whole number of 8-column chunks, or of 32-column steps
+    torch = torch_dev
+    g = torch.Generator(device="cuda").manual_seed(rows + hidden)
+
+    def wide(*shape):
+        e = torch.randint(-40, 40, shape, device="cuda", generator=g).float()
+        return torch.randn(*shape, device="cuda", generator=g) * torch.exp2(e)
+
+    table, x = wide(vocab, hidden), wide(rows, hidden)
+    table[-1, -1], table[0, 0], x[-1, 5] = float("inf"), float("nan"), float("-inf")
+    got = {}
+    for form in (None, "0", "1", "2"):
+        tuning("LOOM_AMD_LM_ROWS", form)
+        got[form] = tf.lm_head(table, x, sequential)
+    tuning("LOOM_AMD_LM_ROWS", None)
+    one = torch.cat([tf.lm_head(table, x[r:r + 1].clone(), sequential) for r in range(rows)])
+    for form, logits in got.items():
+        assert torch.equal(logits.isnan(), one.isnan()), form
+        assert torch.equal(logits.nan_to_num(0.5), one.nan_to_num(0.5)), form
+
+
 @pytest.mark.parametrize("norm", ["strict", "fast"])
 @pytest.mark.parametrize("hidden,heads,inter,seq", [(2560, 20, 6912, 40), (256, 4, 516, 5)])
 def test_block_row_norm_workgroups_agree(orc, torch_dev, tf, tuning, norm, hidden, heads, inter, seq):

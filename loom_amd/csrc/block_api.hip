@@ -789,16 +789,31 @@ void loom_amd_model_release(loom_amd_model* m) {
 
 // Whether a greedy head of `batch` rows screens them one after another (the
 // int8 codes once a row) or forms every logit in one pass over the fp32 table.
-// Measured in us on gfx950 (hidden 2560; x = entries over those of vocab
-// 128256): a screened row 28 + 50 x (three short launches and the codes), the
-// full head of 2 to 16 rows and its pick 20 + 298 x (630 x in sequential
-// order), of one row 20 + 195 x and more than the screened row for every table
-// that a model has.
+// A decode step of a one-layer model on gfx950, us, full head and screened:
+//   hidden 2560, vocab  8,000   32,000   64,000   96,000   128,256
+//     1 row             140/93   144/94  153/100  221/108  245/114
+//     2 rows           106/165  140/164  211/172  281/189  351/207
+//     3 rows           114/226  149/227  220/236  290/262  362/287
+//     4 rows           105/268  138/268  210/285  281/321  352/352
+//   hidden 1024: 2 rows 75/89, 88/99, 116/105, 144/110, 168/121; 3 rows 121/138
+//     at 64,000, 173/163 at 128,256; 4 rows 179/202 at 128,256
+// One row is always screened (measured from 1,000 entries and hidden 256 on;
+// slower only in sequential order on a small table, 158 against 134 at 2,000 x
+// 2560).  For more, the terms below are fitted to these steps: a screened row
+// costs the exact logits of its candidates (by hidden, the sequential chain
+// more) and the codes, the full head a round of the chip or the table's bytes
+// (two row tiles from 17 rows on; sequential order a pass for each of the first
+// rows or the chains' rounds).
 static bool head_screens(const loom_amd_model* m, int batch) {
-    if (!m->lm_q || tune_int("LOOM_AMD_LM_SCREEN", 1) == 0) return false;
-    if (batch == 1) return true;
-    const double x = (double)m->vocab * m->hidden / (128256.0 * 2560.0);
-    return batch * (28.0 + 50.0 * x) <= 20.0 + (m->lm_sequential ? 630.0 : 298.0) * x * ceil_div(batch, 16);
+    const int mode = tune_int("LOOM_AMD_LM_SCREEN", 1);
+    if (!m->lm_q || mode == 0) return false;
+    if (batch == 1 || mode == 2) return true;
+    const double h = m->hidden, u = m->vocab / 128256.0, x = u * h / 2560.0;
+    const int passes = ceil_div(batch, 32);
+    const double row = 5.0 + (m->lm_sequential ? 0.032 : 0.0185) * h + 9.0 * u + 13.0 * x;
+    const double full = 10.0 + (m->lm_sequential ? max(0.031 * h, min(240.0 * batch, 630.0 * passes) * x)
+                                                 : max(0.0148 * h, (batch > 16 ? 380.0 * passes : 285.0) * x));
+    return batch * row <= full;
 }
 
 // Final norm + LM head + argmax of each sequence's last row (row stride ld

@@ -2597,11 +2597,33 @@ hipError_t launch_attention_rope(const int32_t* acc, const float* amax, float sq
     return hipGetLastError();
 }
 
-// Strict prefill tiles (heads x query tiles x sequences) up to which the two
-// launches are shorter (the BitNet-2B block, one launch against two: 80 tiles
-// 143 -> 129 us, 160 188 -> 161, 320 291 -> 252; 640 equal, 1,280 1,668 against
-// 1,734).
+// Whether strict prefill attention takes the two launches: `tiles` is heads x
+// query tiles x sequences.  The value launch forms the probabilities again and
+// the score launch cuts a tile's chunks of 32 positions in four, so few chunks or
+// a grid that fills the chip by itself are shorter in one launch.  A strict block on gfx950, us, one launch -> two:
+//   head size 128, 20 heads: 1 x 17 80.5 -> 80.6, 1 x 33 99.8 -> 97.3, 1 x 64
+//   118 -> 112, 2 x 64 127 -> 125, 4 x 33 127 -> 129, 4 x 64 137 -> 139, 8 x 33
+//   165 -> 170; from 97 positions 1 x 97 139 -> 128, 4 x 100 195 -> 186, 1 x 512
+//   278 -> 241; 640 tiles equal, 1,280 1,668 -> 1,734
+//   head size 64, 16 heads (no column cut): 1 x 33 74.3 -> 76.5, 1 x 64 89.2 ->
+//   89.6, 2 x 17 71.2 -> 73.5, 4 x 64 102 -> 104, 4 x 100 (256 tiles) 121 -> 123;
+//   1 x 97 105 -> 103, 2 x 130 122 -> 120, 1 x 384 162 -> 150, 1 x 700 234 -> 218
+// A decode step of more than 16 rows has a tile per head and row and a position
+// that the host does not know here, at most the span (two layers, 24 steps, ms):
+//   head size 128, 20 heads, from position 120: 17 rows 9.0 -> 8.9, 20 rows 9.2 ->
+//   9.8, 25 rows 9.6 -> 10.4; from 500: 20.0 -> 18.2, 20.7 -> 21.0, 22.2 -> 23.2
+//   head size 64, 16 heads, from 120: 17 rows 5.84 -> 5.81, 25 rows 6.06 -> 6.23;
+//   from 500: 11.4 -> 10.6, 12.3 -> 12.0, 32 rows equal
 constexpr int kSplitTiles = 512;
+
+static bool attention_splits(long tiles, int seq, int span, int hd) {
+    if (const int forced = tune_int("LOOM_AMD_ATTN_SPLIT", -1); forced >= 0) return tiles <= forced;
+    if (seq == 1) return tiles <= (hd == 128 ? 352 : 400) && span > 256;
+    const int positions = seq;  // (a call of several tokens starts at position 0)
+    if (tiles > kSplitTiles || positions <= 32) return false;
+    if (positions <= 64) return hd == 128 && tiles <= 80;
+    return positions > 128 || hd == 128 || tiles <= 200;
+}
 
 hipError_t launch_attention(const double* q, const float* cache_k, const float* cache_v,
                             int batch, int seq, const int* pos0, int msl, int span, int heads,
@@ -2680,7 +2702,7 @@ hipError_t launch_attention(const double* q, const float* cache_k, const float* 
 #define LAMD_FAST(HDV, QTV)                                                                          \
     hipLaunchKernelGGL((attn_tile_mfma_kernel<HDV, QTV>), gridf, dim3(256), 0, s, q, cache_k, cache_v, \
                        pos0, msl, span, heads, kv_heads, seq, scratch, out)
-        if (strict && (long)grid.x * grid.y * grid.z <= tune_int("LOOM_AMD_ATTN_SPLIT", kSplitTiles)) {
+        if (strict && attention_splits((long)grid.x * grid.y * grid.z, seq, span, hd)) {
             double* pm = scratch + (size_t)rows * heads * span;
             const dim3 ga(heads, grid.y, batch * kScoreParts), gb(heads * (hd / 64), grid.y, batch);
 #define LAMD_SPLIT(HDV)                                                                                         \

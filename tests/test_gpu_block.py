@@ -909,6 +909,30 @@ def test_model_sequential_lm_head(orc, torch_dev, tf):
     model.release()
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("batch,msl", [(17, 300), (17, 96), (48, 300)])
+def test_strict_decode_of_many_rows_forms_agree(orc, torch_dev, tf, tuning, hd, batch, msl):
+    # more than 16 rows a step: in two launches (few tiles, a long cache), in one,
+    # and forced either way the same bytes
+    torch = torch_dev
+    sh = Shape(256, 8, 4, hd, 512, msl)
+    w = Weights(orc, sh, seed=1801, act=ACT_SILU)
+    cfg = w.cfg(tf, "strict")
+    cfg.max_batch = batch
+    gw = w.gpu(tf)
+    x_in = orc.normal_f32(batch * 40 * sh.hidden, 1802).reshape(batch, 40, sh.hidden)
+    step = orc.normal_f32(batch * sh.hidden, 1803).reshape(batch, 1, sh.hidden)
+    outs = {}
+    for split in (None, str(1 << 20), "0"):
+        tuning("LOOM_AMD_ATTN_SPLIT", split)
+        blk = tf.BitNetBlock(cfg, gw)
+        blk.forward(to_dev(torch, x_in))
+        y, t = blk.forward(to_dev(torch, step), taps=True)
+        outs[split] = (y.cpu().numpy().tobytes(), t.attn.cpu().numpy().tobytes())
+        blk.release()
+    assert outs[None] == outs["0"] == outs[str(1 << 20)]
+
+
 @pytest.mark.parametrize("sequential", [False, True])
 @pytest.mark.parametrize("rows,vocab,hidden,skip", [(2, 65, 32, 0), (16, 63, 136, 0), (17, 130, 260, 0), (33, 64, 257, 0),
                                                     (5, 1, 9, 0), (4, 300, 512, 1), (18, 999, 520, 4)])

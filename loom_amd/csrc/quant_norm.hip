@@ -1,5 +1,6 @@
 // quant_norm.hip -- weight repack, activation quantization and the SwiGLU
 // inner RMSNorm + requantization (gfx950).
+#include <climits>
 #include <type_traits>
 
 #include "device_common.hpp"
@@ -814,12 +815,33 @@ __global__ __launch_bounds__(W * 64) void row_norm_block_kernel(RowNormArgs a) {
     }
 }
 
+// Rows up to which the W-wave kernel is shorter than the 256-thread kernels.  Its
+// 512 threads are idle beyond a group of four columns each and fewer workgroups
+// share a CU, so many narrow rows are not.  One launch on gfx950, us, 256 threads
+// -> eight waves:
+//   RMSNorm, fast: 1,024 columns 150 rows 4.8 -> 4.7, 300 5.5 -> 5.9, 850 5.5 ->
+//   7.3; 1,536 500 rows 6.3 -> 5.7, 700 6.5 -> 6.7; 2,048 700 rows 7.2 -> 6.8,
+//   850 7.4 -> 7.9; 2,560 1,000 rows 8.8 -> 8.4; strict alike (1,024 columns, 300
+//   rows 7.8 -> 8.7); 512 columns none
+//   inner norms: 512 columns 150 rows 4.2 -> 4.2, 300 4.3 -> 4.5; 1,024 500 rows
+//   5.4 -> 5.1, 700 5.4 -> 5.8; 1,536 700 rows 6.2 -> 6.2 (fp64 strict 11.4 ->
+//   10.6), 850 6.5 -> 7.0; 2,048 850 rows 7.8 -> 7.1 (fp64 strict 14.2 -> 15.1)
+//   sixteen waves: shorter up to 1,000 rows, but for RMSNorm, fast, just above
+//   4,096 columns (4,160: 700 rows 11.4 -> 11.3, 850 12.0 -> 13.9)
+static int row_block_max_rows(int kind, int strict, int n) {
+    if (n > kRowBlockWide) return kind == kRowRms && !strict ? (n - 3072) * 7 / 10 : INT_MAX;
+    return kind == kRowRms ? (n - 768) * 6 / 10 : (n - 256) / 2;
+}
+
 // Launches the W-wave kernel and returns true, or returns false (nothing
 // launched) when the rows do not qualify: n % 4 != 0, rows or outputs not
-// 16-byte aligned, totals already formed, or LOOM_AMD_ROWNORM_BLOCK=0.
+// 16-byte aligned, totals already formed, or more rows than the kernel is
+// shorter for (LOOM_AMD_ROWNORM_BLOCK=1 takes any number, 0 none).
 bool launch_row_norm_block(int kind, int strict, const RowNormArgs& a, hipStream_t s, hipError_t* e) {
-    if (tune_int("LOOM_AMD_ROWNORM_BLOCK", 1) == 0 || a.totals) return false;
+    const int mode = tune_int("LOOM_AMD_ROWNORM_BLOCK", 2);
+    if (mode == 0 || a.totals) return false;
     if (a.m <= 0 || a.n <= 0 || a.n % 4 != 0 || a.n > kMaxNormCols || (strict && a.n > kMaxStrictNormCols)) return false;
+    if (mode != 1 && a.m > row_block_max_rows(kind, strict, a.n)) return false;
     if (a.xq && (a.ldq % 4 != 0 || a.ldq < a.n || ((uintptr_t)a.xq & 3) != 0)) return false;
     const size_t es = kind == kRowInnerF64 ? 8 : 4;
     auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };

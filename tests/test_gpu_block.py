@@ -1009,6 +1009,30 @@ def test_block_row_norm_workgroups_agree(orc, torch_dev, tf, tuning, norm, hidde
     assert outs[1] == outs[0]
 
 
+@pytest.mark.parametrize("norm", ["strict", "fast"])
+@pytest.mark.parametrize("hidden,heads", [(4160, 65), (6400, 50), (8064, 63)])
+def test_block_wide_row_norm_workgroups_agree(orc, torch_dev, tf, tuning, norm, hidden, heads):
+    # RMSNorm and the fp64 inner norm of rows above 4,096 columns: sixteen waves,
+    # each step of the ordered sum's terms per lane, up to the widest strict row
+    # (64 KB of LDS for its values): every tap is the bytes of the 256-thread
+    # kernels
+    torch = torch_dev
+    sh = Shape(hidden, heads, heads, hidden // heads, 64, 64)
+    w = Weights(orc, sh, seed=1521, act=ACT_SILU)
+    gw = w.gpu(tf)
+    x_in = orc.normal_f32(3 * hidden, 1522).reshape(3, hidden)
+    outs = {}
+    for block in (1, 0):
+        tuning("LOOM_AMD_ROWNORM_BLOCK", block)
+        blk = tf.BitNetBlock(w.cfg(tf, norm), gw)
+        x = to_dev(torch, x_in)
+        _, t = blk.forward(x, taps=True)
+        torch.cuda.synchronize()
+        outs[block] = [x.cpu().numpy().tobytes()] + [a.tobytes() for a in t.numpy().values()]
+        blk.release()
+    assert outs[1] == outs[0]
+
+
 @pytest.mark.parametrize("hd", [32, 128])
 @pytest.mark.parametrize("prompt", [2, 30, 62, 126, 254, 318])
 def test_strict_decode_chains_at_chunk_edges(orc, torch_dev, tf, hd, prompt):

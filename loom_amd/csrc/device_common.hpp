@@ -491,11 +491,11 @@ struct OrderedSumLds {
 };
 
 // Terms per lane of ordered_sum_block for n terms over 64W threads: the
-// smallest of 3, 5, 11, 15, 27, 33 that covers n (odd, so the lanes' blocks
+// smallest of 3, 5, 11, 15, 17, 27, 33 that covers n (odd, so the lanes' blocks
 // start in different LDS banks).
 __host__ __device__ constexpr int ordered_sum_lane_terms(int n, int w) {
     const int need = (n + 64 * w - 1) / (64 * w);
-    return need <= 3 ? 3 : need <= 5 ? 5 : need <= 11 ? 11 : need <= 15 ? 15 : need <= 27 ? 27 : 33;
+    return need <= 3 ? 3 : need <= 5 ? 5 : need <= 11 ? 11 : need <= 15 ? 15 : need <= 17 ? 17 : need <= 27 ? 27 : 33;
 }
 
 // ordered_sum_block for G terms a lane, which get(i) (0 <= i < n) returns; every
@@ -699,6 +699,7 @@ __device__ __forceinline__ double ordered_sum_block(const double* t, int n, doub
     if (G == 11) return ordered_sum_core<W, 11>(get, n, s0, sh);
     if (G == 15) return ordered_sum_core<W, 15>(get, n, s0, sh);
     if constexpr (kMax > 27) {
+        if (G == 17) return ordered_sum_core<W, 17>(get, n, s0, sh);
         if (G == 27) return ordered_sum_core<W, 27>(get, n, s0, sh);
     }
     return ordered_sum_core<W, kMax>(get, n, s0, sh);

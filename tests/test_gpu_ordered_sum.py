@@ -158,6 +158,16 @@ def test_ordered_sum_rows_negative_start(torch_dev, n, threads):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,threads", [(3840, 256), (3841, 256), (4352, 256), (4353, 256), (7680, 512), (7681, 512), (8000, 512)])
+def test_ordered_sum_rows_lane_term_steps(torch_dev, n, threads):
+    # either side of the seventeen terms a lane, on four and eight waves
+    rng = np.random.default_rng(n)
+    for kind in ("squares", "squares_fine", "ties", "sparse", "mixed_sign", "nan"):
+        t = rows_of_kind(kind, n, rng)
+        assert same_bits(gpu_ordered_sums(torch_dev, t, 0.0, threads), sequential(t, 0.0)), kind
+
+
+@pytest.mark.gpu
 def test_ordered_sum_rows_many_rows(torch_dev):
     # BitNet-2B widths, 512 rows each (the strict norms' inputs: fp32 squares)
     rng = np.random.default_rng(3)

@@ -173,7 +173,7 @@ __global__ __launch_bounds__(256 * KW, 2) void gemm_lds_kernel(MatArgs p, GemmGr
     const int tid = threadIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
-    const int wn = wave & 3, kw = wave >> 2;  // weight rows; K half of every stage (KW = 2)
+    const int wn = KW == 1 ? wave : wave & 3, kw = KW == 1 ? 0 : wave >> 2;  // weight rows; K half of every stage
     const int l32 = lane & 31, h = lane >> 5;
     const int M = p.e.m;
     const int ktiles = p.ktiles;
@@ -386,6 +386,7 @@ __global__ __launch_bounds__(256 * KW, 2) void gemm_lds_kernel(MatArgs p, GemmGr
         // stage buffers (block i in buffer i; integer sums, so exact in any
         // order) and are done
         __builtin_amdgcn_s_barrier();  // every wave has read its last stage
+        __asm__ __volatile__("" ::: "memory");
         v4i* const x0 = (v4i*)As0 + wn * 256 + lane;
         v4i* const x1 = (v4i*)As1 + wn * 256 + lane;
         if (kw == 1) {
@@ -762,10 +763,13 @@ constexpr int kMaxSplit = 4;
 // Eight waves a half-width tile, each four on one K half of every stage, where
 // the workgroups do not share their CUs (at most kHalfKMaxTiles) and K is long:
 // with four waves a CU one wave a SIMD waits out every operand read and
-// barrier, about 1,000 cycles a stage of 512 MFMA cycles.  N = 2560, K = 6912:
-// 300 rows 15.7 -> 14.3 us, 512 rows 15.5 -> 14.0 (two more stages of prefetch
-// instead: no change).  At K = 2560 both take the same, at K = 1000 the halves'
-// exchange costs 0.3 us, hence kHalfKMinKtiles.
+// barrier, about 1,000 cycles a stage of 512 MFMA cycles.  N = 2560, us, four
+// waves -> eight: K = 6912 at 300 rows 21.3 -> 19.9 with its quantization, 512
+// rows 22.6 -> 21.0; K = 4096 (16 tiles) 15.9 -> 15.0 and 16.4 -> 15.4; over K
+// 4,096 to 10,240, N 1,280 to 3,840 and 130 to 512 rows 0 to 8 % less, none more
+// (two more stages of prefetch instead: no change).  At K = 2560 both take the
+// same, at K = 1000 the halves' exchange costs 0.3 us; between 10 and 16 tiles
+// it was not measured, hence kHalfKMinKtiles.
 constexpr int kHalfKMaxTiles = 256;
 constexpr int kHalfKMinKtiles = 16;
 

@@ -896,6 +896,19 @@ def test_gemm_k_halves(orc, torch_dev, bn, tuning, rows, cols, M):
     _check_dense(orc, torch_dev, bn, m, x, activation=0, residual=res)
 
 
+@pytest.mark.parametrize("rows,cols,M", [(130, 4000, 65), (512, 4300, 129), (1000, 4608, 300), (2560, 6912, 512)])
+def test_gemm_four_wave_half_width_tiles_on_long_k(orc, torch_dev, bn, tuning, rows, cols, M):
+    # the same sizes on four waves a tile, the form above 256 tiles
+    tuning("LOOM_AMD_GEMM_NJ", "1")
+    tuning("LOOM_AMD_GEMM_SPLIT", "1")
+    tuning("LOOM_AMD_GEMM_KHALF", "0")
+    m = orc.random_matrix(rows, cols, seed=rows + cols + M)
+    x = orc.normal_f32(M * cols, seed=M + 21).reshape(M, cols)
+    res = orc.normal_f32(M * rows, seed=M + 22).reshape(M, rows)
+    _check_dense(orc, torch_dev, bn, m, x)
+    _check_dense(orc, torch_dev, bn, m, x, activation=0, residual=res)
+
+
 @pytest.mark.parametrize("n", [2560, 6912, 1000, 260, 8192, 4, 1001])
 def test_norm_quant_rows_one_wave_equal_workgroup(orc, torch_dev, bn, tuning, n):
     # fast inner norm + requantization of 1024 or more rows, one wave per row,

@@ -327,12 +327,6 @@ __device__ __forceinline__ double wave_scan_f64_dpp(double v) {
     return v;
 }
 
-// a wave-uniform 64-bit value (e.g. read from LDS) into scalar registers
-__device__ __forceinline__ unsigned long long uniform_u64(unsigned long long v) {
-    return ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
-           (unsigned)__builtin_amdgcn_readfirstlane((int)v);
-}
-
 __device__ __forceinline__ double readlane_d(double v, int lane) {
     const long long b = __double_as_longlong(v);
     const int lo = __builtin_amdgcn_readlane((int)b, lane);

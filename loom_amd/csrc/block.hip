@@ -2306,15 +2306,19 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const int* __restrict
 // are -0, which leaves a sum as it is, so wave 0 adds whole groups of 32.
 // What bounds it: for one row the chains (7.5 cycles an addition), for several
 // the rounds of workgroups.  One row takes DG = 16, C = 256 (74 KB of LDS, two
-// workgroups a CU), more rows DG = 32, C = 64 (36 KB, four a CU), so eight rows
+// workgroups a CU), a grid of more rows DG = 32, C = 64 (36 KB, four a CU), so eight rows
 // of 20 heads are one round instead of two and a half.  A strict decode layer
 // at BitNet-2B shape (gfx950, us; the head's share included): one row at 2,048
 // positions 98.5 with a branch in every sixteen additions and barriers that
 // wait for the loads, 87.3 now (90.2 with DG = 32); two rows 92.4 with DG = 32,
 // 106.3 with DG = 16; eight rows at 120 positions 86 -> 82, at 2,048 151 -> 130.
+// Up to 256 workgroups of DG = 16 are one a CU, and its longer chunks are the
+// shorter walk of a long cache (this launch, 16 heads of 64, two rows: position
+// 2,000 20.6 -> 17.8, 500 8.8 -> 8.5; at 60 4.8 -> about 5.5), so they are taken
+// for a span of more than 512, which is all that the host knows.
 // grid (heads * HD / DG, rows), 320 threads.
 constexpr int kChainDepth = 4;
-constexpr int kChainWideRows = 2;
+constexpr int kChainNarrowGrid = 256, kChainNarrowSpan = 512;
 constexpr int kChainThreads = 320;  // wave 0: the chains; waves 1-4: loads, probabilities, products
 
 template <int HD, int DG, int C>
@@ -2516,7 +2520,7 @@ static hipError_t launch_strict_decode(const double* q, float* cache_k, float* c
                                        const RopeArgs& ra, double* out, hipStream_t s) {
     const int nc = attn_nchunk(span);
     const dim3 gs(kv_heads, nc, rows), t(256);
-    const bool wide = rows >= kChainWideRows;
+    const bool wide = rows > 1 && (heads * hd / 16 * rows > kChainNarrowGrid || span <= kChainNarrowSpan);
 #define LAMD_SCORES(HDV)                                                                          \
     {                                                                                             \
         if (ra.acc && (ra.qk.q || ra.qk.k))                                                       \

@@ -1060,6 +1060,31 @@ def test_strict_decode_chains_at_chunk_edges(orc, torch_dev, tf, hd, prompt):
     one.release()
 
 
+@pytest.mark.parametrize("hd,rows", [(32, 3), (64, 2), (128, 9)])
+@pytest.mark.parametrize("prompt", [254, 510, 700])
+def test_strict_decode_chains_of_several_rows_in_a_long_cache(orc, torch_dev, tf, hd, rows, prompt):
+    # a span above 512: several rows on one grid of the 256-position chunks (and
+    # nine rows of four heads of 128, too many for one), the bits of one row each
+    torch = torch_dev
+    sh = Shape(256, 4, 2, hd, 512, 720)
+    w = Weights(orc, sh, seed=1611, act=ACT_SILU)
+    gw = w.gpu(tf)
+    cfg = w.cfg(tf, "strict")
+    cfg.max_batch = rows
+    both, one = tf.BitNetBlock(cfg, gw), tf.BitNetBlock(cfg, gw)
+    x = orc.normal_f32(rows * prompt * sh.hidden, 1612 + prompt).reshape(rows, prompt, sh.hidden)
+    steps = orc.normal_f32(4 * rows * sh.hidden, 1613).reshape(4, rows, 1, sh.hidden)
+    both.forward(to_dev(torch, x))
+    got = [both.forward(to_dev(torch, s))[0].cpu().numpy() for s in steps]
+    for b in range(rows):
+        one.forward(to_dev(torch, x[b:b + 1]))
+        for s, g in zip(steps, got):
+            r = one.forward(to_dev(torch, s[b:b + 1]))[0].cpu().numpy()
+            assert g[b].tobytes() == r[0].tobytes()
+    both.release()
+    one.release()
+
+
 @pytest.mark.parametrize("hd", [64, 128])
 @pytest.mark.parametrize("batch,seq", [(1, 17), (1, 32), (2, 33), (1, 97), (2, 160)])
 def test_strict_prefill_two_launches_equal_one(orc, torch_dev, tf, tuning, hd, batch, seq):

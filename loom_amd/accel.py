@@ -100,6 +100,7 @@ class CompiledLayer:
         self._h = handle
         self._in = in_b
         self._out = out_b
+        self._spare = []  # an input copy's buffer, kept from one call for the next
 
     def in_bytes(self) -> int:
         return self._in
@@ -117,8 +118,13 @@ class CompiledLayer:
             raise AccelError(f"accel: buffer size mismatch in={inv.nbytes} want={self._in} "
                              f"out={outv.nbytes} want={self._out}")
         # copied while the GIL is held: the call may wait for another layer's,
-        # and the caller may refill its array meanwhile
-        in_buf = (C.c_char * inv.nbytes).from_buffer_copy(inv)
+        # and the caller may refill its array meanwhile (each call that runs at
+        # the same time has a buffer of its own)
+        try:
+            in_buf = self._spare.pop()
+        except IndexError:
+            in_buf = (C.c_char * self._in)()
+        memoryview(in_buf).cast("B")[:] = inv
         out_buf = (C.c_char * outv.nbytes).from_buffer(outv) if not outv.readonly else None
         if out_buf is None:
             raise AccelError("accel: output buffer is read-only")
@@ -127,6 +133,8 @@ class CompiledLayer:
         rc = self._api.loom_accel_infer(self._h, C.addressof(in_buf), inv.nbytes,
                                         C.addressof(out_buf), outv.nbytes, C.byref(ms), err,
                                         ERR_BUF)
+        if not self._spare:
+            self._spare.append(in_buf)
         if rc != 0:
             raise AccelError(f"accel: infer: {err.value.decode(errors='replace')}")
         return InferResult(ms.value)
@@ -135,6 +143,7 @@ class CompiledLayer:
         if self._h is not None:
             self._api.loom_accel_release_layer(self._h)
             self._h = None
+            self._spare.clear()
 
 
 class Plugin:

@@ -129,6 +129,34 @@ def test_infer_copies_its_input_when_called():
     assert out.tolist() == [0.0, 1.0, 2.0, 3.0]
 
 
+def test_infer_of_two_calls_at_once_keeps_their_inputs_apart():
+    # a call that starts while another runs (played by an API that calls back)
+    # copies its input beside the first one's, whose buffer a later call reuses
+    import numpy as np
+    from loom_amd import accel
+
+    first, second = np.full(4, 1.0, np.float32), np.full(4, 2.0, np.float32)
+    out, out2, at = np.zeros(4, np.float32), np.zeros(4, np.float32), []
+
+    class Api:
+        depth = 0
+
+        def loom_accel_infer(self, handle, inp, in_bytes, outp, out_bytes, ms, err, err_len):
+            at.append(inp)
+            Api.depth += 1
+            if Api.depth == 1:
+                layer.infer(second, out2)
+            C.memmove(outp, inp, out_bytes)
+            return 0
+
+    layer = accel.CompiledLayer(Api(), 1, first.nbytes, out.nbytes)
+    layer.infer(first, out)
+    assert at[0] != at[1]
+    assert out.tolist() == [1.0] * 4 and out2.tolist() == [2.0] * 4
+    layer.infer(second, out)
+    assert out.tolist() == [2.0] * 4
+
+
 def test_c_loader_conformance(amd_lib, tmp_path):
     from loom_amd import _lib
     exe = tmp_path / "abi_conformance"

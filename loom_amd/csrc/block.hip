@@ -3226,8 +3226,9 @@ __global__ __launch_bounds__(256) void lm_head_rows_kernel(const float* __restri
 //    table too (2560 575 -> 634, 448 102 -> 129) unless a multiple of 1,024
 //    floats apart (1024 279 -> 261, 2048 570 -> 492), up to four of narrow rows
 //    (hidden 128, 32,000: 11.5 -> 15.7),
-//  - and short rows of a small table while each workgroup has a CU (hidden 1024,
-//    4,000 30 -> 34; 576, 8,000 20 -> 22; 2560, three rows 83 -> 75).
+//  - and short rows of a small table while each workgroup has a CU (hidden 448,
+//    8,000 17 -> 20 with the table from memory, 15 -> 18 from the caches; 576 21
+//    -> 24, 20 -> 22; at 768 27 -> 28, at 1024 36 -> 35 and 35 -> 34).
 static int head_rows_tile(int vocab, int hidden, int rows, bool dottile, bool vec) {
     constexpr int kCus = 256;
     if (rows < 2) return 0;
@@ -3239,8 +3240,7 @@ static int head_rows_tile(int vocab, int hidden, int rows, bool dottile, bool ve
         if (rows == 2 && ceil_div(vocab, 64) > kCus + kCus / 8) tiles = 0;
         if (rows == 3 && large && hidden % 64 == 0 && hidden % 1024 != 0) tiles = 0;
         if (rows <= 4 && hidden >= 128 && hidden <= 256) tiles = 0;
-        if (hidden <= 1024 && vocab <= (hidden <= 640 ? 8192 : 6000) && rows * ceil_div(vocab, kHeadLogits) <= kCus)
-            tiles = 0;
+        if (hidden <= 640 && hidden % 64 == 0 && vocab <= 8192 && rows * ceil_div(vocab, kHeadLogits) <= kCus) tiles = 0;
     }
     return min(max(tune_int("LOOM_AMD_LM_ROWS", tiles), 0), 2);
 }

@@ -830,7 +830,7 @@ __global__ __launch_bounds__(W * 64) void row_norm_block_kernel(RowNormArgs a) {
 //   4,096 columns (4,160: 700 rows 11.4 -> 11.3, 850 12.0 -> 13.9)
 static int row_block_max_rows(int kind, int strict, int n) {
     if (n > kRowBlockWide) return kind == kRowRms && !strict ? (n - 3072) * 7 / 10 : INT_MAX;
-    return kind == kRowRms ? (n - 768) * 6 / 10 : (n - 256) / 2;
+    return kind == kRowRms ? (n - 684) * 6 / 10 : (n - 256) / 2;
 }
 
 // Launches the W-wave kernel and returns true, or returns false (nothing

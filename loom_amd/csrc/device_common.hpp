@@ -680,22 +680,24 @@ __device__ __forceinline__ double ordered_sum_core(Get get, int n, double s0, Or
 // branch per kind took 7,100 (about 220 cycles a record beside its additions,
 // 7.5 cycles each), one with the checks in fp64 9,900; sixteen waves of half
 // the terms walk 34 records in 4,170 cycles and wait longer for each other.
-template <int W>
+// LO and HI bound n where a caller knows it (steps outside are left out).
+template <int W, int LO = 1, int HI = kMaxStrictNormCols>
 __device__ __forceinline__ double ordered_sum_block(const double* t, int n, double s0,
                                                    OrderedSumLds<W>& sh) {
     static_assert(W == 4 || W == 8, "the sum runs on four or eight waves");
     if (n <= 0) return s0;
     const auto get = [t](int i) { return t[i]; };
     const int G = ordered_sum_lane_terms(n, W);
-    constexpr int kMax = ordered_sum_lane_terms(kMaxStrictNormCols, W);
-    if (G == 3) return ordered_sum_core<W, 3>(get, n, s0, sh);
-    if (G == 5) return ordered_sum_core<W, 5>(get, n, s0, sh);
-    if (G == 11) return ordered_sum_core<W, 11>(get, n, s0, sh);
-    if (G == 15) return ordered_sum_core<W, 15>(get, n, s0, sh);
-    if constexpr (kMax > 27) {
-        if (G == 17) return ordered_sum_core<W, 17>(get, n, s0, sh);
-        if (G == 27) return ordered_sum_core<W, 27>(get, n, s0, sh);
-    }
+    constexpr int kMin = ordered_sum_lane_terms(LO, W), kMax = ordered_sum_lane_terms(HI, W);
+#define LAMD_SUM_STEP(g) \
+    if constexpr (kMin <= (g) && (g) < kMax) if (G == (g)) return ordered_sum_core<W, (g)>(get, n, s0, sh);
+    LAMD_SUM_STEP(3)
+    LAMD_SUM_STEP(5)
+    LAMD_SUM_STEP(11)
+    LAMD_SUM_STEP(15)
+    LAMD_SUM_STEP(17)
+    LAMD_SUM_STEP(27)
+#undef LAMD_SUM_STEP
     return ordered_sum_core<W, kMax>(get, n, s0, sh);
 }
 

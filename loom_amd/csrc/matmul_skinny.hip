@@ -280,9 +280,9 @@ __global__ __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(2)))
                         OrderedSumLds<4> w4;
                     } osum;
                     if (k >= kSumWideCols) {
-                        tot[0] = ordered_sum_block<8>(sq, k, 0.0, osum.w8);
+                        tot[0] = ordered_sum_block<8, kSumWideCols>(sq, k, 0.0, osum.w8);
                     } else {
-                        tot[0] = ordered_sum_block<4>(sq, k, 0.0, osum.w4);
+                        tot[0] = ordered_sum_block<4, 1, kSumWideCols - 1>(sq, k, 0.0, osum.w4);
                     }
                 } else if constexpr (WAVES >= 4) {
                     __shared__ OrderedSumLds<4> osum;
